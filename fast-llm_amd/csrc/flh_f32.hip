@@ -10,7 +10,9 @@
 //    dot_row_fast / dot_row_fast_q8_0 / dot_row_fast_dequant, bitwise: the
 //    256-element chunk formats (Q4_K, Q6_K -- the reference GPU masks' Q6_K
 //    route --, Q5_0, IQ2_XXS, IQ3_XXS) on one wave per row (k_dot_fastk),
-//    F32 (e.g. an MoE router) and Q8_0 on 16 lanes per row (k_dot_f32row).
+//    Q8_0 and several columns of a large F32 matrix on 16 lanes per row
+//    (k_dot_f32row), other F32 (e.g. an MoE router) on a workgroup per row
+//    (k_dot_f32small).
 //  * ROUTER_SEL / SILU_MUL / WMERGE / MERGE: the reference's single-thread
 //    canonical ops (src/runtime/decode_params.h:234-295,
 //    runtime_internal.h:274-281), one thread per token / element.  expf is
@@ -631,6 +633,93 @@ __global__ __launch_bounds__(256) void k_dot_f32row(DotArgs a, uint32_t T) {
     }
 }
 
+// F32 rows, one column, or a small matrix (an MoE router) and any: one
+// workgroup per (row, group of up to 4 columns).  k_dot_f32row gives a small
+// matrix 16 rows per workgroup -- a handful of workgroups, each waiting for a
+// chain of load round trips (8 x 4096: 10.3 us, 26 us with 4 columns).  Here
+// every element of a tile of up to 4096 columns is requested at once (16-byte
+// loads, all 256 threads), the products go to LDS as P[column][j][m] (element
+// 16 m + j), and lane (column, j) of wave 0 adds its L[j] over m: the same
+// products and the same order of additions, bit for bit.  What is left is one
+// memory round trip and the 256 dependent additions of a 4096-column row
+// (about 1 us): 8 x 4096 3.5 us, 4.5 us with 8 columns.  The row pitch M + 4 (M a multiple of 64) spreads a 16-byte
+// read of the 16 j over all 64 banks.
+constexpr uint32_t F32S_T = 4096;                                 // columns per tile
+constexpr uint32_t F32S_MP = F32S_T / 16 + 4;                     // pitch of P in floats
+
+template <int NXT>
+__global__ __launch_bounds__(256) void k_dot_f32small(DotArgs a) {
+    extern __shared__ __align__(16) uint8_t f32r_smem[];
+    float * P = reinterpret_cast<float *>(f32r_smem);             // [NXT][16][F32S_MP]
+    const uint32_t tid = threadIdx.x, lane = tid & 63, j = lane & 15, c = lane >> 4;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t r = blockIdx.x, p0 = blockIdx.y * NXT, nx = min((uint32_t)NXT, a.nx - p0);
+    const uint32_t cols = a.cols, n16 = cols & ~15u;
+    const float * w = reinterpret_cast<const float *>(a.w + (a.id_slot ? (size_t)(*a.id_slot) * a.estride : 0)) +
+                      (size_t)r * cols;
+    const float * x = a.x + (size_t)p0 * a.xstride;
+    float * y = a.y + (size_t)p0 * a.ystride + r;
+    const bool mine = wave == 0 && c < nx;                        // this lane runs a chain
+    const float yv = mine && j == 0 ? y[(size_t)c * a.ystride] : 0.f;
+    u32x4 wv[4], xv[NXT][4];
+    auto fetch = [&](uint32_t c0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const uint32_t k = c0 + 4 * (tid + 256 * q);          // n16 % 16 == 0: four elements in or out
+            if (k < n16) {
+                wv[q] = *(const u32x4 *)(w + k);
+#pragma unroll
+                for (int p = 0; p < NXT; ++p)
+                    if ((uint32_t)p < nx) xv[p][q] = *(const u32x4 *)(x + (size_t)p * a.xstride + k);
+            }
+        }
+    };
+    float L = 0.f;
+    if (n16) fetch(0);
+    for (uint32_t c0 = 0; c0 < n16; c0 += F32S_T) {
+        if (c0) __syncthreads();                                  // the chain has read the last tile
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const uint32_t e = 4 * (tid + 256 * q), k = c0 + e;
+            if (k < n16) {
+#pragma unroll
+                for (int p = 0; p < NXT; ++p)
+                    if ((uint32_t)p < nx)
+#pragma unroll
+                        for (int i = 0; i < 4; ++i)
+                            P[(p * 16 + (e & 15) + i) * F32S_MP + (e >> 4)] =
+                                __uint_as_float(wv[q][i]) * __uint_as_float(xv[p][q][i]);
+            }
+        }
+        __syncthreads();
+        if (c0 + F32S_T < n16) fetch(c0 + F32S_T);
+        if (mine) {
+            const float * q = P + (size_t)(c * 16 + j) * F32S_MP;
+            const uint32_t M = min(F32S_T, n16 - c0) / 16;
+            uint32_t m = 0;
+            for (; m + 16 <= M; m += 16) {
+                float4 v[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) v[i] = *reinterpret_cast<const float4 *>(q + m + 4 * i);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) { L = L + v[i].x; L = L + v[i].y; L = L + v[i].z; L = L + v[i].w; }
+            }
+            for (; m < M; ++m) L = L + q[m];
+        }
+    }
+    if (!mine) return;
+    const float u = L + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(L), 0x104, 0xF, 0xF, true));
+    const float t = u + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(u), 0x108, 0xF, 0xF, true));
+    const float h2 = t + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(t), 0x101, 0xF, 0xF, true));
+    const float head = h2 + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(h2), 0x102, 0xF, 0xF, true));
+    if (j == 0) {
+        float tail = 0.f;
+        const float * xc = x + (size_t)c * a.xstride;
+        for (uint32_t k = n16; k < cols; ++k) tail = tail + w[k] * xc[k];
+        y[(size_t)c * a.ystride] = yv + (head + tail);
+    }
+}
+
 __global__ void k_dot_canon(int fmt, DotArgs a) {
     const uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= (uint64_t)a.rows * a.nx) return;
@@ -647,6 +736,15 @@ __global__ void k_dot_canon(int fmt, DotArgs a) {
     *y = *y + v;
 }
 
+// Workgroups (rows x groups of 4 columns) up to which several columns of an
+// F32 matrix take k_dot_f32small, every column group reading the row anew.
+// k_dot_f32row / k_dot_f32small, us: 64 x 2048 with 4 columns 13.9 / 3.4, with
+// 16 55 / 3.5, 8 x 4096 with 8 49 / 4.5, 1024 x 4096 with 4 26 / 11.5, 2048 x
+// 1024 with 4 9.8 / 8.3; 4096 x 4096 with 4 29 / 35, 16384 x 1024 with 4 21 / 55.
+// One column takes it at any size: 8 x 4096 10.3 / 3.5, 4096 x 4096 18.8 /
+// 14.3, 16384 x 4096 58 / 46, 16384 x 1024 18.2 / 17.7.
+constexpr uint64_t F32S_MAX_WG = 2048;
+
 static int launch_f32(bool fast, int fmt, const DotArgs & a, hipStream_t s) {
     if (fmt < FMT_F32 || fmt > FMT_IQ3_XXS)
         return set_error(FLH_ERR_UNSUPPORTED, "fp32 dot: format not supported");
@@ -654,6 +752,20 @@ static int launch_f32(bool fast, int fmt, const DotArgs & a, hipStream_t s) {
     if (n == 0) return FLH_OK;
     const bool chunked = fmt == FMT_Q4_K || fmt == FMT_Q6_K || fmt == FMT_Q5_0 || fmt == FMT_IQ2_XXS ||
                          fmt == FMT_IQ3_XXS;
+    // F32, one column or a small matrix: one workgroup per row and group of 4
+    // columns, all columns in one launch
+    if (fast && fmt == FMT_F32 && a.nx <= 16 && a.rows <= 0x7FFFFFFFu &&
+        (a.nx == 1 || (uint64_t)a.rows * ((a.nx + 3) / 4) <= F32S_MAX_WG)) {
+        const uint32_t nxt = a.nx == 1 ? 1 : a.nx == 2 ? 2 : 4;
+        const size_t smem = (size_t)nxt * 16 * F32S_MP * 4;
+        const void * kern = nxt == 1 ? (const void *)k_dot_f32small<1> : nxt == 2 ? (const void *)k_dot_f32small<2>
+                                                                               : (const void *)k_dot_f32small<4>;
+        if (int rc = lds_fits(kern, smem, "k_dot_f32small")) return rc;
+        (void)hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
+        void * args[] = {const_cast<DotArgs *>(&a)};
+        return hip_check(hipLaunchKernel(kern, dim3(a.rows, (a.nx + nxt - 1) / nxt), dim3(256), args, smem, s),
+                         "k_dot_f32small launch");
+    }
     if (fast && (chunked || fmt == FMT_F32 || fmt == FMT_Q8_0) && a.nx > 4 && a.nx <= 16) {
         // more than 4 columns: groups of 4, each its own pass over the weights
         // (per column the 4-column launch costs least: the activation tiles of
@@ -698,7 +810,7 @@ static int launch_f32(bool fast, int fmt, const DotArgs & a, hipStream_t s) {
         const dim3 gw((a.rows + 15) / 16);
         const uint32_t slots = a.nx == 1 ? 0 : a.nx == 2 ? 1 : 2;
         static const void * const kf32[3] = {
-            (const void *)k_dot_f32row<FMT_F32, 1, 4>, (const void *)k_dot_f32row<FMT_F32, 2, 4>,
+            (const void *)k_dot_f32row<FMT_F32, 2, 4>, (const void *)k_dot_f32row<FMT_F32, 2, 4>,
             (const void *)k_dot_f32row<FMT_F32, 4, 2>};
         static const void * const kq8[3] = {
             (const void *)k_dot_f32row<FMT_Q8_0, 1, 4>, (const void *)k_dot_f32row<FMT_Q8_0, 2, 4>,
