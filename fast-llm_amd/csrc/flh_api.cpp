@@ -248,6 +248,37 @@ static int validate_table(const flh_task * t, uint32_t n) {
     return FLH_OK;
 }
 
+// Row tiles of one matrix that follow task i of a table (a dot: a holds its
+// arguments) join its launch: a.rows grows and i moves to the last one.  The
+// graph builder cuts every matrix into such tiles; a fused launch (norm and
+// quantisation in front of its dot) takes them too, or the rest of the matrix
+// would be a second launch that finds the weight stream drained (decoder layer
+// of 1024 columns in tiles of 512 rows: 8 launches a layer instead of 5).  A
+// tile whose output lies over what the launch reads (the activation column and
+// its appendices; the columns nx0, nx1 of a fused norm) stays out: its launch
+// of its own would have come after those reads.
+static void merge_tiles(const flh_task * t, uint32_t n, uint32_t & i, DotArgs & a, const float * nx0 = nullptr,
+                        const float * nx1 = nullptr) {
+    const flh_task & k = t[i];
+    auto over = [&](const float * y, uint32_t rows, const float * x, size_t bytes) {
+        return x && (const uint8_t *)y < (const uint8_t *)x + bytes && (const uint8_t *)x < (const uint8_t *)(y + rows);
+    };
+    while (i + 1 < n) {
+        const flh_task & q = t[i + 1];
+        if (q.kind != k.kind || q.fmt != k.fmt || q.cols != k.cols || q.x != k.x || (q.nx ? q.nx : 1u) != a.nx ||
+            q.xstride != k.xstride || q.ystride != k.ystride || q.aux != k.aux || q.aux2 != k.aux2 ||
+            (const uint8_t *)q.w != a.w + (uint64_t)a.rows * flh_row_bytes(k.fmt, k.cols) ||
+            (float *)q.y != a.y + a.rows || (a.nx > 1 && a.rows + q.rows > k.ystride))
+            return;
+        if (a.nx == 1 && (over((const float *)q.y, q.rows, a.x, x_alloc_bytes(a.cols)) ||
+                          over((const float *)q.y, q.rows, nx0, (size_t)a.cols * 4) ||
+                          over((const float *)q.y, q.rows, nx1, (size_t)a.cols * 4)))
+            return;
+        a.rows += q.rows;
+        ++i;
+    }
+}
+
 }  // namespace flh
 
 using namespace flh;
@@ -516,18 +547,7 @@ int flh_exec_tasks(const flh_task * t, uint32_t n, int fast, uint32_t i8_mask, u
                 DotArgs a{(const uint8_t *)k.w, idx ? (const uint32_t *)k.aux : nullptr, idx ? k.aux2 : 0,
                           (const float *)k.x, (float *)k.y, k.rows, k.cols, k.nx ? k.nx : 1u,
                           k.xstride, k.ystride};
-                // fuse following row tiles of the same matrix into this launch
-                while (i + 1 < n) {
-                    const flh_task & q = t[i + 1];
-                    if (q.kind != k.kind || q.fmt != k.fmt || q.cols != k.cols || q.x != k.x ||
-                        (q.nx ? q.nx : 1u) != a.nx || q.xstride != k.xstride || q.ystride != k.ystride ||
-                        q.aux != k.aux || q.aux2 != k.aux2 ||
-                        (const uint8_t *)q.w != a.w + (uint64_t)a.rows * flh_row_bytes(k.fmt, k.cols) ||
-                        (float *)q.y != a.y + a.rows || (a.nx > 1 && a.rows + q.rows > k.ystride))
-                        break;
-                    a.rows += q.rows;
-                    ++i;
-                }
+                merge_tiles(t, n, i, a);
                 rc = dispatch_dot(k.fmt, a, fast, i8_mask, i8k_mask, s);
                 break;
             }
@@ -542,9 +562,11 @@ int flh_exec_tasks(const flh_task * t, uint32_t n, int fast, uint32_t i8_mask, u
                     (q->fmt == FLH_FMT_Q4_K || q->fmt == FLH_FMT_Q6_K) && ((i8k_mask >> q->fmt) & 1u)) {
                     DotArgs a{(const uint8_t *)q->w, nullptr, 0, (const float *)q->x, (float *)q->y,
                               q->rows, q->cols, 1u, q->xstride, q->ystride};
+                    uint32_t last = i + 1;
+                    merge_tiles(t, n, last, a);
                     rc = launch_act_dot_kstream(q->fmt, a, s);
                     if (rc != FLH_ERR_UNSUPPORTED) {
-                        ++i;
+                        i = last;
                         break;
                     }
                 }
@@ -570,8 +592,9 @@ int flh_exec_tasks(const flh_task * t, uint32_t n, int fast, uint32_t i8_mask, u
                     !((uintptr_t)p.wnorm & 15)) {
                     DotArgs a{(const uint8_t *)d->w, nullptr, 0, (const float *)d->x, (float *)d->y, d->rows, d->cols,
                               1u, d->xstride, d->ystride};
-                    rc = rmsnorm_dot(d->fmt, a, NormArgs{p.x, p.wnorm, p.eps}, fast, i8_mask, i8k_mask, s);
                     i += 2;
+                    merge_tiles(t, n, i, a, p.x, p.wnorm);
+                    rc = rmsnorm_dot(d->fmt, a, NormArgs{p.x, p.wnorm, p.eps}, fast, i8_mask, i8k_mask, s);
                     break;
                 }
                 rc = launch_rmsnorm_act_q8(p.x, p.wnorm, p.y, p.n, p.eps, fuse, s);
