@@ -178,78 +178,158 @@ int launch_act_q8(float * x, void * y_q81, uint32_t cols, uint32_t nx,
 }
 
 // ---------------------------------------------------------------- dequant --
-// Bit-exact restatement of dequant_chunk's value formulas; byte loads (this
-// is a correctness/embedding path, not the streamed hot loop).  One thread
-// per 32 outputs (Q8_0: a block; Q4_K: 16 nibble pairs; Q6_K: 16 positions x
-// 4 groups... split as 32 outputs of one group pair).
-__global__ void k_dequant(int fmt, const uint8_t * __restrict__ w, uint32_t rows,
-                          uint32_t cols, float * __restrict__ out) {
-    const uint64_t units_per_row = cols / 32;
-    const uint64_t u = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (u >= units_per_row * rows) return;
-    const uint32_t r = (uint32_t)(u / units_per_row), j = (uint32_t)(u % units_per_row);
-    float * o = out + (size_t)r * cols;
-    if (fmt == FMT_Q8_0) {
-        const uint8_t * b = w + (size_t)r * (cols / 32) * 34 + (size_t)j * 34;
-        const float d = h2f(b[0] | (b[1] << 8));
-        for (int i = 0; i < 32; ++i) o[32 * j + i] = d * (float)(int8_t)b[2 + i];
-    } else if (fmt == FMT_Q5_0) {
-        const uint8_t * b = w + (size_t)r * (cols / 32) * 22 + (size_t)j * 22;
-        const float d = h2f(b[0] | (b[1] << 8));
-        const uint32_t qh = b[2] | (b[3] << 8) | (b[4] << 16) | ((uint32_t)b[5] << 24);
-        for (int i = 0; i < 16; ++i) {
-            const uint32_t lo = (b[6 + i] & 0x0F) | (((qh >> i) << 4) & 0x10);
-            const uint32_t hi = (b[6 + i] >> 4) | ((qh >> (i + 12)) & 0x10);
-            o[32 * j + i] = d * (float)((int)lo - 16);
-            o[32 * j + 16 + i] = d * (float)((int)hi - 16);
-        }
-    } else if (fmt == FMT_Q4_K) {
-        const uint32_t sb = j >> 3, g = j & 7, c = g >> 1;   // group g of superblock sb
-        const uint8_t * b = w + (size_t)r * (cols / 256) * 144 + (size_t)sb * 144;
-        const float d = h2f(b[0] | (b[1] << 8)), dmin = h2f(b[2] | (b[3] << 8));
-        const uint8_t * s = b + 4;
-        uint32_t sc, mn;
-        if (g < 4) { sc = s[g] & 63; mn = s[g + 4] & 63; }
-        else { sc = (s[g + 4] & 0xF) | ((s[g - 4] >> 6) << 4); mn = (s[g + 4] >> 4) | ((s[g] >> 6) << 4); }
-        const float d1 = d * (float)sc, m1 = dmin * (float)mn;
-        const uint8_t * q = b + 16 + 32 * c;
-        float * oo = o + 256 * sb + 64 * c + 32 * (g & 1);
-        for (int l = 0; l < 32; ++l) {
-            const uint32_t nib = (g & 1) ? (q[l] >> 4) : (q[l] & 0xF);
-            oo[l] = d1 * (float)nib - m1;
-        }
-    } else if (fmt == FMT_IQ2_XXS || fmt == FMT_IQ3_XXS) {
-        // group ib of superblock sb: db * (+-grid magnitude), the factor the
-        // reference's canonical IQ dots multiply x by (quants.h:252-254,
-        // 280-283); its dequant_chunk has no IQ case (kernels.h:215-221)
-        const uint32_t sb = j >> 3, ib = j & 7, bb = iq_block_bytes(fmt);
-        const uint8_t * b = w + (size_t)r * (cols / 256) * bb + (size_t)sb * bb;
-        const uint32_t w1 = iq_w1(fmt, b, ib);
-        const float db = iq_db(fmt, h2f(b[0] | (b[1] << 8)), w1);
-        for (int e = 0; e < 32; ++e) o[32 * j + e] = db * (float)iq_val(fmt, b, ib, w1, e);
-    } else {  // Q6_K: group (h, gg) of superblock sb, positions l < 32
-        const uint32_t sb = j >> 3, h = (j >> 2) & 1, gg = j & 3;
-        const uint8_t * b = w + (size_t)r * (cols / 256) * 210 + (size_t)sb * 210;
-        const float d = h2f(b[208] | (b[209] << 8));
-        const uint8_t * ql = b + 64 * h, * qh = b + 128 + 32 * h;
-        const int8_t * sc = (const int8_t *)(b + 192) + 8 * h;
-        float * oo = o + 256 * sb + 128 * h + 32 * gg;
-        for (int l = 0; l < 32; ++l) {
-            const uint8_t lb = ql[l + 32 * (gg & 1)];
-            const int q6 = ((gg < 2) ? (lb & 0xF) : (lb >> 4)) | (((qh[l] >> (2 * gg)) & 3) << 4);
-            oo[l] = d * (float)sc[l / 16 + 2 * gg] * (float)(q6 - 32);
+// Bit-exact restatement of dequant_chunk's value formulas.  A matrix is one
+// array of blocks (rows are whole blocks), so the work is split flat: a unit
+// is 256 outputs (a superblock, or eight 32-weight blocks), lane i of a wave
+// makes outputs 4i..4i+3 of it from one 4-byte read of the quants, so a wave
+// stores 1 KiB in one piece and its reads of a block fall in one or two lines
+// (one thread per 32 outputs stored 4 bytes every 128: 14336 x 4096 of Q4_K
+// took 100 us, 2.7 TB/s).  Bound by the output's 4 bytes per weight: the
+// stores are nontemporal (the output is far larger than an L2; ordinary ones
+// take 64 us, these 40-43 us, 6.3-7.0 TB/s in every format), and a wave makes
+// DEQ_UN = 2 units at once (1: 40-48 us, 4: 42, 8: 46; 1000 x 2048: 3.6 / 3.7
+// / 4.5 / 6.6 us for 1 / 2 / 4 / 8).  Blocks are 2-byte aligned at best, and a
+// caller's address may be odd: the reads are unaligned ones (memcpy), which
+// gfx950 does in one instruction.
+constexpr uint32_t DEQ_UN = 2;
+
+__device__ __forceinline__ uint32_t ldu32(const uint8_t * p) {
+    uint32_t v;
+    __builtin_memcpy(&v, p, 4);
+    return v;
+}
+__device__ __forceinline__ uint32_t ldu16(const uint8_t * p) {
+    uint16_t v;
+    __builtin_memcpy(&v, p, 2);
+    return v;
+}
+// what lane `lane` reads of unit u (e: the lane's first element in its block or superblock)
+struct DeqIn { uint32_t q, a, b, c; };
+
+template <int FMT>
+__device__ __forceinline__ DeqIn deq_load(const uint8_t * w, uint64_t u, uint32_t lane) {
+    DeqIn in{0, 0, 0, 0};
+    const uint32_t e = 4 * lane;
+    if constexpr (FMT == FMT_Q8_0 || FMT == FMT_Q5_0) {
+        constexpr uint32_t BB = FMT == FMT_Q8_0 ? 34 : 22;
+        const uint8_t * b = w + (u * 8 + (lane >> 3)) * BB;
+        const uint32_t i = e & 31;
+        in.a = ldu16(b);
+        if constexpr (FMT == FMT_Q8_0) in.q = ldu32(b + 2 + i);
+        else { in.q = ldu32(b + 6 + (i & 15)); in.b = ldu32(b + 2); }
+    } else if constexpr (FMT == FMT_Q4_K) {
+        const uint8_t * b = w + u * 144;
+        const uint32_t g = lane >> 3;                             // group of 32
+        in.a = ldu32(b);                                          // d | dmin
+        in.q = ldu32(b + 16 + 32 * (g >> 1) + (e & 31));
+        in.b = ldu32(b + 4 + (g & 4 ? 8 : 0));                    // g < 4: scales 0..3, else bytes 8..11
+        in.c = g & 4 ? (b[4 + (g & 3)] | ((uint32_t)b[8 + (g & 3)] << 8)) : b[8 + (g & 3)];
+    } else if constexpr (FMT == FMT_Q6_K) {
+        const uint8_t * b = w + u * 210;
+        const uint32_t h = lane >> 5, gg = (lane >> 3) & 3, l = e & 31;
+        in.q = ldu32(b + 64 * h + l + 32 * (gg & 1));
+        in.b = ldu32(b + 128 + 32 * h + l);
+        in.a = ldu16(b + 208);
+        in.c = b[192 + 8 * h + l / 16 + 2 * gg];
+    } else {
+        const uint8_t * b = w + u * iq_block_bytes(FMT);
+        const uint32_t ib = lane >> 3, l = (e & 31) >> 3;         // group, 8-element run
+        in.a = ldu16(b);
+        if constexpr (FMT == FMT_IQ2_XXS) {
+            in.b = ldu32(b + 2 + 8 * ib + 4);
+            in.q = (uint32_t)(k_iq2_grid[b[2 + 8 * ib + l]] >> (8 * (e & 4)));
+        } else {
+            in.b = ldu32(b + 66 + 4 * ib);
+            in.q = k_iq3_grid[b[2 + 8 * ib + 2 * l + ((e >> 2) & 1)]];
         }
     }
+    return in;
+}
+template <int FMT>
+__device__ __forceinline__ float4 deq_vals(const DeqIn & in, uint32_t lane) {
+    float v[4];
+    const uint32_t e = 4 * lane;
+    if constexpr (FMT == FMT_Q8_0) {
+        const float d = h2f(in.a);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = d * (float)(int8_t)(in.q >> (8 * i));
+    } else if constexpr (FMT == FMT_Q5_0) {
+        const float d = h2f(in.a);
+        const uint32_t s = e & 31, nib = (in.q >> (s & 16 ? 4 : 0)) & 0x0F0F0F0Fu, hb = in.b >> s;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t q5 = ((nib >> (8 * i)) & 0xFu) | (((hb >> i) & 1u) << 4);
+            v[i] = d * (float)((int)q5 - 16);
+        }
+    } else if constexpr (FMT == FMT_Q4_K) {
+        const float d = h2f(in.a & 0xFFFFu), dmin = h2f(in.a >> 16);
+        const uint32_t g = lane >> 3, k = g & 3, s8 = (in.b >> (8 * k)) & 0xFFu;
+        // the 6-bit scale and min of group g from bytes g, g + 4 (g < 4) or g + 4, g - 4, g
+        uint32_t sc, mn;
+        if (g < 4) { sc = s8 & 63u; mn = in.c & 63u; }
+        else { sc = (s8 & 0xFu) | (((in.c & 0xFFu) >> 6) << 4); mn = (s8 >> 4) | ((in.c >> 14) << 4); }
+        const float d1 = d * (float)sc, m1 = dmin * (float)mn;
+        const uint32_t nib = (g & 1) ? (in.q >> 4) & 0x0F0F0F0Fu : in.q & 0x0F0F0F0Fu;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = d1 * (float)((nib >> (8 * i)) & 0xFFu) - m1;
+    } else if constexpr (FMT == FMT_Q6_K) {
+        const float d = h2f(in.a);
+        const uint32_t gg = (lane >> 3) & 3;
+        const uint32_t lo = gg < 2 ? in.q & 0x0F0F0F0Fu : (in.q >> 4) & 0x0F0F0F0Fu;
+        const uint32_t q6 = lo | (((in.b >> (2 * gg)) & 0x03030303u) << 4);
+        const float ds = d * (float)(int8_t)in.c;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = ds * (float)((int)((q6 >> (8 * i)) & 0xFFu) - 32);
+    } else {
+        // db * (+-grid magnitude), the factor the reference's canonical IQ dots
+        // multiply x by (quants.h:252-254, 280-283); its dequant_chunk has no
+        // IQ case (kernels.h:215-221)
+        const float db = iq_db(FMT, h2f(in.a), in.b);
+        const uint32_t sg = iq_sign8(in.b >> (7 * ((e & 31) >> 3))) >> (e & 4);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int m = (int)((in.q >> (8 * i)) & 0xFFu);
+            v[i] = db * (float)((sg >> i) & 1u ? -m : m);
+        }
+    }
+    return make_float4(v[0], v[1], v[2], v[3]);
+}
+// units of 256 outputs; n32: 32-weight blocks in the matrix (the last unit of
+// a 32-weight-block format may be partial: its lanes past the end stop)
+template <int FMT>
+__global__ __launch_bounds__(256) void k_dequant(const uint8_t * __restrict__ w, uint64_t n32, float * __restrict__ out) {
+    typedef float f4a __attribute__((ext_vector_type(4), aligned(4)));
+    const uint32_t lane = threadIdx.x & 63;
+    const uint64_t u0 = ((uint64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * DEQ_UN;
+    DeqIn in[DEQ_UN];
+#pragma unroll
+    for (uint32_t k = 0; k < DEQ_UN; ++k)
+        if ((u0 + k) * 8 + (lane >> 3) < n32) in[k] = deq_load<FMT>(w, u0 + k, lane);
+#pragma unroll
+    for (uint32_t k = 0; k < DEQ_UN; ++k)
+        if ((u0 + k) * 8 + (lane >> 3) < n32) {
+            const float4 v = deq_vals<FMT>(in[k], lane);
+            __builtin_nontemporal_store((f4a{v.x, v.y, v.z, v.w}), reinterpret_cast<f4a *>(out + (u0 + k) * 256 + 4 * lane));
+        }
 }
 
 int launch_dequant(int fmt, const uint8_t * w, uint32_t rows, uint32_t cols,
                    float * out, hipStream_t s) {
     if (fmt < FMT_Q8_0 || fmt > FMT_IQ3_XXS)
         return set_error(FLH_ERR_UNSUPPORTED, "dequant: format not supported");
-    const uint64_t units = (uint64_t)rows * (cols / 32);
-    if (units == 0) return FLH_OK;
-    hipLaunchKernelGGL(k_dequant, dim3((uint32_t)((units + 255) / 256)), dim3(256), 0, s,
-                       fmt, w, rows, cols, out);
+    const uint64_t n32 = (uint64_t)rows * (cols / 32);
+    if (n32 == 0) return FLH_OK;
+    const uint64_t nwg = (n32 + 8 * 4 * DEQ_UN - 1) / (8 * 4 * DEQ_UN);
+    if (nwg > 0x7FFFFFFFull) return set_error(FLH_ERR_UNSUPPORTED, "dequant: more than 2^43 outputs");
+    const dim3 g((uint32_t)nwg), b(256);
+    switch (fmt) {
+        case FMT_Q8_0: hipLaunchKernelGGL(k_dequant<FMT_Q8_0>, g, b, 0, s, w, n32, out); break;
+        case FMT_Q5_0: hipLaunchKernelGGL(k_dequant<FMT_Q5_0>, g, b, 0, s, w, n32, out); break;
+        case FMT_Q4_K: hipLaunchKernelGGL(k_dequant<FMT_Q4_K>, g, b, 0, s, w, n32, out); break;
+        case FMT_Q6_K: hipLaunchKernelGGL(k_dequant<FMT_Q6_K>, g, b, 0, s, w, n32, out); break;
+        case FMT_IQ2_XXS: hipLaunchKernelGGL(k_dequant<FMT_IQ2_XXS>, g, b, 0, s, w, n32, out); break;
+        default: hipLaunchKernelGGL(k_dequant<FMT_IQ3_XXS>, g, b, 0, s, w, n32, out); break;
+    }
     return hip_check(hipGetLastError(), "k_dequant launch");
 }
 
