@@ -133,11 +133,13 @@ void load_tune() {
     if (const char * e = getenv("FLH_MFMA_MIN_COLS")) t.mf_min_cols = (uint32_t)atoi(e);
     if (const char * e = getenv("FLH_NO_MFMA")) t.no_mfma = atoi(e) != 0;
     if (const char * e = getenv("FLH_NO_Q6MF")) t.no_q6mf = atoi(e) != 0;
-    if (const char * e = getenv("FLH_Q6MF_MIN")) {
-        unsigned r = 0, c = 0;
-        if (sscanf(e, "%u,%u", &r, &c) == 2) { t.q6mf_rows = r; t.q6mf_cols = c; }
-    }
     if (const char * e = getenv("FLH_SBL_NX_DEP")) t.sbl_nx_dep = (uint32_t)atoi(e);
+    if (const char * e = getenv("FLH_CW")) {
+        unsigned m = 0, w = 0;
+        if (sscanf(e, "%u,%u", &m, &w) >= 1) { t.cw = m; t.cw_wpc = w; }
+    }
+    for (const char * v : {"FLH_MFMA_PRO", "FLH_MFMA_TUNE", "FLH_MFMA_XC", "FLH_MFMA_OWN", "FLH_MFMA_MIN_COLS"})
+        t.mf_forced = t.mf_forced || getenv(v);
     if (const char * e = getenv("FLH_GGUF_THREADS")) t.gguf_threads = (uint32_t)strtoul(e, nullptr, 0);
     if (const char * e = getenv("FLH_SBL")) {
         unsigned on = 1, w = 0, g = 0, m = 0, pre = 0;
@@ -157,6 +159,11 @@ static int dispatch_dot(int fmt, const DotArgs & a, int fast, uint32_t i8_mask, 
     if ((fmt == FLH_FMT_Q4_K || fmt == FLH_FMT_Q6_K) && ((i8k_mask >> fmt) & 1u))
         return launch_dot_i8k(fmt, a, s);
     if (fmt != FLH_FMT_F32 && ((i8_mask >> fmt) & 1u)) {
+        // several columns of Q8_0 / Q5_0: the matrix cores where they win
+        if (a.nx >= 2 && (fmt == FLH_FMT_Q8_0 || fmt == FLH_FMT_Q5_0)) {
+            const int rc = launch_dot_cw(fmt, a, s);
+            if (rc != FLH_ERR_UNSUPPORTED) return rc;
+        }
         // 2..8 columns of the 32-weight-block formats: one weight pass on the
         // superblock-per-lane layout where its LDS plan fits
         if (a.nx >= 2 && tune().sbl &&
@@ -182,9 +189,10 @@ static int dispatch_dot(int fmt, const DotArgs & a, int fast, uint32_t i8_mask, 
 }
 
 // Grouped expert dots of the 32-weight-block formats (Q8_0, Q5_0, IQ2_XXS,
-// IQ3_XXS x q8_1): the routed superblock-per-lane launch, one workgroup row
-// per (token, slot) pair (the reference runs these per pair too,
-// src/model/decoder.cpp:941-996).  Shapes its LDS plan cannot hold (rows of
+// IQ3_XXS x q8_1).  Q8_0 and Q5_0 of several tokens: the matrix cores, an
+// expert's weights streamed once for all of its pairs.  Otherwise the routed
+// superblock-per-lane launch, one workgroup row per (token, slot) pair (the
+// reference runs these per pair too, src/model/decoder.cpp:941-996).  Shapes its LDS plan cannot hold (rows of
 // more than ~14.5K columns, weights or x not 16-byte aligned) run as the
 // reference's own per-pair STREAM_DOT_IDX tiles, the id read on the device,
 // on the q8_1 int8 path the routed launch computes (same bits); there the
@@ -193,7 +201,9 @@ static int dispatch_dot(int fmt, const DotArgs & a, int fast, uint32_t i8_mask, 
 static int launch_moe_b32(int fmt, const MoeArgs & a, hipStream_t s) {
     if (a.rows == 0 || a.ntok == 0 || a.top_k == 0) return FLH_OK;
     if (a.ntok * a.top_k > 256) return set_error(FLH_ERR_UNSUPPORTED, "moe: ntok*top_k > 256");
-    const int rc = launch_moe_sbl(fmt, a, s);
+    int rc = FLH_ERR_UNSUPPORTED;
+    if (a.ntok > 1) rc = launch_moe_cw(fmt, a, s);
+    if (rc == FLH_ERR_UNSUPPORTED) rc = launch_moe_sbl(fmt, a, s);
     if (rc != FLH_ERR_UNSUPPORTED) return rc;
     for (uint32_t p = 0; p < a.ntok * a.top_k; ++p) {
         const uint32_t xi = a.x_per_slot ? p : p / a.top_k;
@@ -677,8 +687,8 @@ int flh_router_moe_dot(int fmt, const void * w, uint64_t estride, uint32_t rows,
         f.rt_scale = scale;
         f.rt_gates = gates;
         int rc = FLH_ERR_UNSUPPORTED;
-        if ((ntok == 1 || !kf) && tune().sbl) rc = launch_moe_sbl(fmt, f, s);
-        if (rc == FLH_ERR_UNSUPPORTED && kf) rc = launch_moe_mfma(fmt, f, s);
+        if (ntok > 1) rc = launch_moe_cw(fmt, f, s);
+        if (rc == FLH_ERR_UNSUPPORTED && (ntok == 1 || !kf) && tune().sbl) rc = launch_moe_sbl(fmt, f, s);
         if (rc == FLH_ERR_UNSUPPORTED && kf) rc = launch_moe_kstream(fmt, f, s);
         if (rc != FLH_ERR_UNSUPPORTED) return rc;
     }

@@ -633,6 +633,10 @@ int launch_dot_i8k(int fmt, const DotArgs & a0, hipStream_t s) {
     if (nsb == 0 || nsb > 64 || (a0.cols & 255))
         return set_error(FLH_ERR_UNSUPPORTED, "i8k dot: cols must be a multiple of 256, <= 16384");
     if (a0.rows == 0 || a0.nx == 0) return FLH_OK;
+    if (a0.nx >= 2) {
+        const int rc = launch_dot_cw(fmt, a0, s);
+        if (rc != FLH_ERR_UNSUPPORTED) return rc;
+    }
     // several Q4_K columns: the int8 matrix-core kernel, all columns in one
     // pass when they fit its LDS plan, else in groups of 8 or 4
     if (fmt == FMT_Q4_K && a0.nx >= mfma_min_cols(a0.cols)) {
@@ -655,26 +659,6 @@ int launch_dot_i8k(int fmt, const DotArgs & a0, hipStream_t s) {
     for (uint32_t p0 = 0, g = 4; p0 < a0.nx; p0 += g) {
         DotArgs a = a0;
         int rc = FLH_ERR_UNSUPPORTED;
-        // 5-8 columns of matrices of 12288 rows or more on the matrix cores
-        // (14336x4096, 8 columns: 26.6 -> 21.8 us; 6144 rows: 14.6 against
-        // 16.8 us, too few tiles); at 2-4 columns the streaming kernel is as
-        // fast or faster
-        if (fmt == FMT_Q6_K && a0.nx - p0 >= 2 && a0.nx - p0 >= tune().q6mf_cols &&
-            a0.rows >= tune().q6mf_rows && !tune().no_q6mf) {
-            a.x = a0.x + (size_t)p0 * a0.xstride;
-            a.y = a0.y + (size_t)p0 * a0.ystride;
-            a.nx = a0.nx - p0 < 16 ? a0.nx - p0 : 16;               // 9-16 columns in one pass where it fits
-            rc = a.nx > 8 ? launch_dot_q6mf(a, s) : FLH_ERR_UNSUPPORTED;
-            if (rc == FLH_ERR_UNSUPPORTED) {
-                a.nx = a0.nx - p0 < 8 ? a0.nx - p0 : 8;
-                rc = launch_dot_q6mf(a, s);
-            }
-            if (rc != FLH_ERR_UNSUPPORTED) {
-                if (rc) return rc;
-                g = a.nx;
-                continue;
-            }
-        }
         if (fmt == FMT_Q6_K && a0.nx - p0 > 4) {                  // 5-8 columns in one streaming pass
             a.nx = a0.nx - p0 < 8 ? a0.nx - p0 : 8;
             a.x = a0.x + (size_t)p0 * a0.xstride;
@@ -733,7 +717,7 @@ int launch_moe_i8k(int fmt, const MoeArgs & a, hipStream_t s) {
     int rc = FLH_ERR_UNSUPPORTED;
     if (a.ntok == 1 && tune().sbl) rc = launch_moe_sbl(fmt, a, s);     // one token: superblock per lane
     if (rc != FLH_ERR_UNSUPPORTED) return rc;
-    rc = launch_moe_mfma(fmt, a, s);
+    if (a.ntok > 1) rc = launch_moe_cw(fmt, a, s);
     if (rc != FLH_ERR_UNSUPPORTED) return rc;
     rc = launch_moe_kstream(fmt, a, s);
     if (rc != FLH_ERR_UNSUPPORTED) return rc;

@@ -1,5 +1,5 @@
 // flh_dot_mfma.hip -- multi-column Q4_K x q8_K row-dots (speculative verify,
-// grouped MoE experts) on gfx950's int8 matrix cores.
+// the shapes flh_dot_cw.hip leaves to it) on gfx950's int8 matrix cores.
 //
 // With several activation columns the per-lane VALU dot of the streaming
 // kernel (flh_dot_kstream.hip) becomes instruction-bound (about 300 wave
@@ -896,55 +896,6 @@ __global__ __launch_bounds__(512) void k_dot_mfma(DotArgs a, uint32_t nrb) {
     mf_body<NC, D, KH, MfColsStrided, XC, OWN>(w, a.rows, a.cols, C, a.nx, nrb, blockIdx.x, gridDim.x, sm);
 }
 
-// Grouped expert matvec (MoE): the routed experts share the grid (moe_assign).  The workgroup collects
-// the (token, slot) pairs routed to e and streams e's weights once per group
-// of NC pairs (the columns); with no pair routed to e it exits before any
-// weight byte is requested.  Column p's activation index and output index
-// sit in LDS tables read with the lane's own (lane-varying) p.
-struct MfColsMoe {
-    const float * x0;
-    float * y0;
-    uint32_t xs, ys;
-    const uint32_t * xi;                      // __shared__ [NC]
-    const uint32_t * yi;                      // __shared__ [NC]
-    __device__ const float * x(uint32_t p) const { return x0 + (size_t)lds_ld32(&xi[p]) * xs; }
-    __device__ float * y(uint32_t p) const { return y0 + (size_t)lds_ld32(&yi[p]) * ys; }
-};
-
-template <int NC, int D, bool KH, bool OWN = false>
-__global__ __launch_bounds__(512) void k_moe_mfma(MoeArgs a, uint32_t nrbp) {
-    extern __shared__ __attribute__((aligned(16))) uint8_t sm[];
-    __shared__ uint32_t pairs[256];
-    __shared__ uint32_t npairs;
-    __shared__ uint32_t cxi[NC], cyi[NC];
-    const uint32_t tid = threadIdx.x;
-    __shared__ uint32_t rids[256];
-    if (tid == 0) npairs = 0;
-    const uint32_t * ids = moe_route(a, rids);
-    uint32_t g, G;
-    const uint32_t e = moe_assign(ids, a.ntok * a.top_k, a.n_expert, blockIdx.y * gridDim.x + blockIdx.x,
-                                  gridDim.x * gridDim.y, g, G);                 // (barriers)
-    if (e >= a.n_expert) return;
-    // pairs i = tok * top_k + slot routed to e (order free: every column's
-    // output is computed independently)
-    if (tid < a.ntok * a.top_k && ids[tid] == e) pairs[atomicAdd(&npairs, 1u)] = tid;
-    __syncthreads();
-    const uint32_t np = npairs;
-    const uint8_t * w = a.w + (size_t)e * a.estride;
-    for (uint32_t p0 = 0; p0 < np; p0 += NC) {
-        const uint32_t nx = min((uint32_t)NC, np - p0);
-        if (tid < NC) {
-            const uint32_t ts = pairs[p0 + (tid < nx ? tid : 0)];
-            cxi[tid] = a.x_per_slot ? ts : ts / a.top_k;
-            cyi[tid] = ts;
-        }
-        __syncthreads();
-        const MfColsMoe C{a.x, a.y, a.xstride, a.ystride, cxi, cyi};
-        mf_body<NC, D, KH, MfColsMoe, false, OWN>(w, a.rows, a.cols, C, nx, nrbp, g, G, sm);
-        __syncthreads();
-    }
-}
-
 // ----------------------------------------------------------------- launch --
 // chunks each wave requests before the activations are staged (the rest of
 // its ring after its first chunk); 0 = the whole ring (measured best here)
@@ -976,8 +927,8 @@ size_t lds_limit();
 // fits.
 template <int NC>
 static int mf_plan_kh(uint32_t rows, uint32_t nsb, uint32_t G, uint32_t & nrb, int & D, bool & kh, size_t & smb,
-                      bool allow_kh = true, bool * xc = nullptr, bool * own = nullptr) {
-    const size_t lim = lds_limit() - 4096;                    // the MoE kernel's static tables
+                      bool * xc = nullptr, bool * own = nullptr) {
+    const size_t lim = lds_limit() - 4096;
     const uint32_t rpw = (rows + G - 1) / G;
     // a batch's old y values are one 64-float DMA per wave: nrb * NC <= 512
     nrb = ((rpw + 15) / 16) * 16;
@@ -990,9 +941,7 @@ static int mf_plan_kh(uint32_t rows, uint32_t nsb, uint32_t G, uint32_t & nrb, i
     if (t.mf_nrb >= 16 && t.mf_nrb % 16 == 0 && t.mf_nrb <= 512 / NC) nrb = t.mf_nrb;
     const int force_kh = t.mf_kh;
     kh = force_kh == 1 || (force_kh != 0 && mf_smem_bytes<NC, false>(16, nsb, 2) > lim);
-    // K halves need at least 8 superblocks per row, and the grouped (MoE)
-    // planner allows them only as a last resort
-    if (kh && (nsb < 8 || (!allow_kh && force_kh != 1))) kh = false;
+    if (kh && nsb < 8) kh = false;                            // K halves need at least 8 superblocks per row
     // one 16-row tile per workgroup where K halves would be needed: the
     // activations ride in the chunks instead (Tune::mf_xc = false: off)
     if (xc) *xc = false;
@@ -1035,9 +984,9 @@ int mfma_plan(uint32_t rows, uint32_t cols, uint32_t nx, uint32_t * out) {
     int D;
     bool kh, xc;
     size_t smb;
-    const int rc = nx <= 4 ? mf_plan_kh<4>(rows, nsb, G, nrb, D, kh, smb, true, &xc)
-                 : nx <= 8 ? mf_plan_kh<8>(rows, nsb, G, nrb, D, kh, smb, true, &xc)
-                           : mf_plan_kh<16>(rows, nsb, G, nrb, D, kh, smb, true, &xc);
+    const int rc = nx <= 4 ? mf_plan_kh<4>(rows, nsb, G, nrb, D, kh, smb, &xc)
+                 : nx <= 8 ? mf_plan_kh<8>(rows, nsb, G, nrb, D, kh, smb, &xc)
+                           : mf_plan_kh<16>(rows, nsb, G, nrb, D, kh, smb, &xc);
     if (rc) return FLH_ERR_UNSUPPORTED;
     out[0] = kh;
     out[1] = xc;
@@ -1055,7 +1004,7 @@ static int mf_launch(const DotArgs & a, hipStream_t s) {
     bool kh;
     size_t smb;
     bool xc, own;
-    if (mf_plan_kh<NC>(a.rows, nsb, G, nrb, D, kh, smb, true, &xc, &own)) return FLH_ERR_UNSUPPORTED;
+    if (mf_plan_kh<NC>(a.rows, nsb, G, nrb, D, kh, smb, &xc, &own)) return FLH_ERR_UNSUPPORTED;
     if (xc) return mf_launch_d<NC, 2, false, true>(a, nrb, G, smb, s);
     if (kh) return mf_launch_d<NC, 2, true>(a, nrb, G, smb, s);
     if (own) return mf_launch_d<NC, 2, false, false, true>(a, nrb, G, smb, s);
@@ -1067,66 +1016,6 @@ static int mf_launch(const DotArgs & a, hipStream_t s) {
 // its registers, cols <= 4096, and slower beyond).
 uint32_t mfma_min_cols(uint32_t cols) {
     return tune().mf_min_cols ? tune().mf_min_cols : (cols > 4096 ? 2u : 3u);
-}
-
-uint32_t mfma_min_cols(uint32_t cols);
-
-template <int NC, int D, bool KH, bool OWN = false>
-static int mf_moe_launch_d(const MoeArgs & a, uint32_t nrb, uint32_t gx, size_t smb, hipStream_t s) {
-    if (moe_rows(a) == 0) return FLH_OK;
-    if (int rc = lds_fits((const void *)k_moe_mfma<NC, D, KH, OWN>, smb, "k_moe_mfma: LDS over the limit")) return rc;
-    (void)hipFuncSetAttribute((const void *)k_moe_mfma<NC, D, KH, OWN>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                              (int)smb);
-    hipLaunchKernelGGL((k_moe_mfma<NC, D, KH, OWN>), dim3(gx, moe_rows(a)), dim3(MF_WAVES * 64), smb, s, a,
-                       nrb | (mf_pro() << 16));
-    return hip_check(hipGetLastError(), "k_moe_mfma launch");
-}
-
-template <int NC>
-static int mf_moe_launch(const MoeArgs & a, hipStream_t s, bool allow_kh) {
-    const uint32_t nsb = a.cols >> 8;
-    // the experts that can be active at once share the CUs (one workgroup each)
-    const uint32_t pairs = a.ntok * a.top_k;
-    const uint32_t active = pairs < a.n_expert ? pairs : a.n_expert;
-    uint32_t gx = ((uint32_t)num_cus() + active - 1) / active;
-    if (gx > a.rows) gx = a.rows;
-    uint32_t nrb;
-    int D;
-    bool kh;
-    size_t smb;
-    bool own;
-    if (mf_plan_kh<NC>(a.rows, nsb, gx, nrb, D, kh, smb, allow_kh, nullptr, &own)) return FLH_ERR_UNSUPPORTED;
-    if (kh) return mf_moe_launch_d<NC, 2, true>(a, nrb, gx, smb, s);
-    if (own) return mf_moe_launch_d<NC, 2, false, true>(a, nrb, gx, smb, s);
-    return D == 2 ? mf_moe_launch_d<NC, 2, false>(a, nrb, gx, smb, s) : mf_moe_launch_d<NC, 3, false>(a, nrb, gx, smb, s);
-}
-
-// Grouped Q4_K expert matvec on the matrix cores for token batches of at
-// least mfma_min_cols(cols) tokens; FLH_ERR_UNSUPPORTED (nothing launched)
-// otherwise or when the shape does not fit.
-int launch_moe_mfma(int fmt, const MoeArgs & a, hipStream_t s) {
-    const uint32_t nsb = a.cols >> 8;
-    if (fmt != FMT_Q4_K || nsb == 0 || (a.cols & 255) || nsb > 64 || a.ntok < mfma_min_cols(a.cols))
-        return FLH_ERR_UNSUPPORTED;
-    if (((uintptr_t)a.w & 15) || (a.estride & 15) || ((uintptr_t)a.x & 3) || (a.xstride & 3) || tune().no_mfma ||
-        a.ntok * a.top_k > 256)
-        return FLH_ERR_UNSUPPORTED;
-    // an expert gets at most one pair per token.  K halves only as a last
-    // resort: most experts get few pairs, and 4-column passes that hold the
-    // whole activations beat an 8-column pass that restages them (Mixtral
-    // top-2 of 8, batch 8: 217 vs 253 us)
-    // 8-column passes only when an active expert averages more than 4 pairs:
-    // a 4-column pass costs ~10 % less per byte, and an expert with more pairs
-    // than that (rare at such averages) takes a second pass (Mixtral top-2 of
-    // 8, batch 8, 2 pairs per expert on average: 209 -> 189 us)
-    const uint32_t pairs = a.ntok * a.top_k, active = pairs < a.n_expert ? pairs : a.n_expert;
-    const bool wide = a.ntok > 4 && (pairs + active - 1) / active > 4;
-    int rc = FLH_ERR_UNSUPPORTED;
-    if (wide) rc = mf_moe_launch<8>(a, s, false);
-    if (rc == FLH_ERR_UNSUPPORTED) rc = mf_moe_launch<4>(a, s, false);
-    if (rc == FLH_ERR_UNSUPPORTED && wide) rc = mf_moe_launch<8>(a, s, true);
-    if (rc == FLH_ERR_UNSUPPORTED) rc = mf_moe_launch<4>(a, s, true);
-    return rc;
 }
 
 // Q4_K x q8_K with 1..16 columns; FLH_ERR_UNSUPPORTED (nothing launched) when

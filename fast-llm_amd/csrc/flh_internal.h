@@ -91,13 +91,16 @@ struct Tune {
     bool mf_own = true;                 // FLH_MFMA_OWN=0: parked terms and a fold pass, not register sums
     uint32_t mf_min_cols = 0;           // FLH_MFMA_MIN_COLS (0: 2 above 4096 columns, else 3)
     bool no_mfma = false;               // FLH_NO_MFMA=1: never the matrix-core kernels
-    bool no_q6mf = false;               // FLH_NO_Q6MF=1: several Q6_K columns off the matrix cores
-    uint32_t q6mf_rows = 12288, q6mf_cols = 5;  // FLH_Q6MF_MIN = "rows,cols": the smallest shape sent there
+    bool no_q6mf = false;               // FLH_NO_Q6MF=1: Q6_K off the matrix cores
     // superblock-per-lane single-column kernel, FLH_SBL = "on,waves,wgs_per_cu,max_wgs,pre"
     // (0 = default; max_wgs caps the grid, for tests of long per-wave chunk
     // lists; pre = waves requesting a chunk before the activation lands, 0: half, 255: all)
     uint32_t sbl = 1, sbl_w = 0, sbl_wpc = 0, sbl_gmax = 0, sbl_pre = 0;
     uint32_t sbl_nx_dep = 0;            // FLH_SBL_NX_DEP: ring stages of the several-column kernel (0: planned)
+    bool mf_forced = false;             // any FLH_MFMA_* override: Q4_K stays on that kernel
+    // chain-per-wave matrix-core kernel, FLH_CW = "mode[,wgs_per_cu]": 0 never,
+    // 1 where it is the faster one, 2 wherever it takes the shape; wgs_per_cu 0: planned
+    uint32_t cw = 1, cw_wpc = 0;
     uint32_t gguf_threads = 0;          // FLH_GGUF_THREADS: host copy threads of an upload (0: all, <= 16)
 };
 const Tune & tune();
@@ -128,8 +131,6 @@ int launch_act_dot_kstream(int fmt, const DotArgs & a, hipStream_t s);
 // Q4_K x q8_K, 1..16 columns, on the int8 matrix cores (flh_dot_mfma.hip);
 // FLH_ERR_UNSUPPORTED (nothing launched) if the shape does not fit its plan
 int launch_dot_mfma(int fmt, const DotArgs & a, hipStream_t s);
-// grouped expert variant (MoE, Q4_K, batches of several tokens)
-int launch_moe_mfma(int fmt, const MoeArgs & a, hipStream_t s);
 // fewest columns for which STREAM_DOT uses launch_dot_mfma
 uint32_t mfma_min_cols(uint32_t cols);
 int mfma_plan(uint32_t rows, uint32_t cols, uint32_t nx, uint32_t * out);
@@ -142,7 +143,12 @@ int launch_dot_fast_f32(int fmt, const DotArgs & a, hipStream_t s);
 int launch_dequant(int fmt, const uint8_t * w, uint32_t rows, uint32_t cols,
                    float * out, hipStream_t s);
 int launch_moe_i8k(int fmt, const MoeArgs & a, hipStream_t s);
-int launch_dot_q6mf(const DotArgs & a, hipStream_t s);
+// 2..16 columns of Q8_0, Q5_0 (q8_1), Q4_K, Q6_K (q8_K) on the int8 matrix
+// cores, one accumulator chain per wave (flh_dot_cw.hip); FLH_ERR_UNSUPPORTED
+// (nothing launched) if the kernel does not take the shape or another is faster
+int launch_dot_cw(int fmt, const DotArgs & a, hipStream_t s);
+// grouped experts on the same kernel (several tokens)
+int launch_moe_cw(int fmt, const MoeArgs & a, hipStream_t s);
 // LDS-staged grouped expert kernel; FLH_ERR_UNSUPPORTED if it does not fit
 int launch_moe_kstream(int fmt, const MoeArgs & a, hipStream_t s);
 int launch_moe_sbl(int fmt, const MoeArgs & a, hipStream_t s);
