@@ -159,8 +159,8 @@ static int dispatch_dot(int fmt, const DotArgs & a, int fast, uint32_t i8_mask, 
     if ((fmt == FLH_FMT_Q4_K || fmt == FLH_FMT_Q6_K) && ((i8k_mask >> fmt) & 1u))
         return launch_dot_i8k(fmt, a, s);
     if (fmt != FLH_FMT_F32 && ((i8_mask >> fmt) & 1u)) {
-        // several columns of Q8_0 / Q5_0: the matrix cores where they win
-        if (a.nx >= 2 && (fmt == FLH_FMT_Q8_0 || fmt == FLH_FMT_Q5_0)) {
+        // Q8_0 / Q5_0: the matrix cores where they win (several columns, wide rows)
+        if (fmt == FLH_FMT_Q8_0 || fmt == FLH_FMT_Q5_0) {
             const int rc = launch_dot_cw(fmt, a, s);
             if (rc != FLH_ERR_UNSUPPORTED) return rc;
         }

@@ -577,7 +577,7 @@ template <int FMT> static int cw_launch(const DotArgs & a, hipStream_t s) {
 }
 
 // Whether a matrix with nx columns is faster here than on the format's other
-// several-column kernel (us here / there):
+// kernel (us here / there):
 //  * Q4_K against k_dot_mfma, whose tiles are 16 x 144-byte pieces but which
 //    stages the columns once per workgroup: 4 columns 14336x4096 9.7 / 10.6,
 //    6144x4096 6.3 / 7.2, 4096x14336 10.0 / 11.7; 8 columns 4096x14336 12.4 /
@@ -595,11 +595,15 @@ template <int FMT> static int cw_launch(const DotArgs & a, hipStream_t s) {
 //    20.6, Q5_0 14336x4096 12.1 / 14.0; 4 columns 15.5 / 18.5, 12.4 / 17.1,
 //    4096x14336 15 / 46; 16 columns 14336x4096 22.7 / 52, 4096x14336 23 / 149.
 //    A few long rows leave most of the chip idle here: Q8_0 1024x2816 with 2 / 4
-//    columns 5.5 / 4.6 and 5.5 / 5.2.
+//    columns 5.5 / 4.6 and 5.5 / 5.2.  One column against k_dot_sbl: rows wider
+//    than its one pass per lane group holds well, Q8_0 4096x14336 14.7 / 18.3,
+//    8192x8192 14.7 / 17.0, Q5_0 27648x5120 22.6 / 32.8; not 14336x4096 15.2 / 13.4,
+//    2048x5632 7.6 / 6.3.
 static bool cw_wins(int fmt, uint32_t rows, uint32_t cols, uint32_t nx) {
     const uint32_t T = (rows + 15) / 16, cus = (uint32_t)num_cus();
     if (fmt == FMT_Q4_K) return nx <= 4 || (nx <= 8 ? rows <= 16384 : T <= cus || cols > 4096);
     if (fmt == FMT_Q6_K) return nx > 2 || cols > 8192;
+    if (nx == 1) return cols > 4096 && T >= cus;
     if (nx <= 4 && 4 * T <= cus && cols > 2048) return false;
     return nx > 2 || fmt == FMT_Q5_0 || cols > 4096;
 }
@@ -610,7 +614,7 @@ static bool cw_on(int fmt) {
 
 int launch_dot_cw(int fmt, const DotArgs & a, hipStream_t s) {
     if (!cw_on(fmt) || (tune().cw == 1 && !cw_wins(fmt, a.rows, a.cols, a.nx))) return FLH_ERR_UNSUPPORTED;
-    if (a.nx < 2 || a.nx > 16 || !cw_takes(fmt, a.w, a.estride, a.x, a.xstride, a.nx, a.cols)) return FLH_ERR_UNSUPPORTED;
+    if (a.nx < 1 || a.nx > 16 || !cw_takes(fmt, a.w, a.estride, a.x, a.xstride, a.nx, a.cols)) return FLH_ERR_UNSUPPORTED;
     if (a.rows == 0) return FLH_OK;
     switch (fmt) {
         case FMT_Q8_0: return cw_launch<FMT_Q8_0>(a, s);

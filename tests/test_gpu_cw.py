@@ -47,6 +47,14 @@ def test_cw_bitwise(flh, orc, gpu, wgs, fmt, rows, cols, nx):
         check(flh, orc, gpu, fmt, rows, cols, nx, pad=nx % 3)
 
 
+@pytest.mark.parametrize("rows,cols", [(4080, 4352), (4081, 4352), (4100, 4096), (4111, 8448), (4097, 14592)])
+@pytest.mark.parametrize("fmt", [Q8_0, Q5_0])
+def test_one_wide_column(flh, orc, gpu, fmt, rows, cols):
+    """One column on either side of the line (more than 4096 columns, a tile per CU)."""
+    say("cw one column", fmt, rows, cols)
+    check(flh, orc, gpu, fmt, rows, cols, 1)
+
+
 @pytest.mark.parametrize("fmt", FMTS)
 def test_cw_expert_slot(flh, orc, gpu, fmt):
     say("cw slot", fmt)
