@@ -7,6 +7,7 @@
 #include <string.h>
 #include <stdlib.h>
 #include <string>
+#include <vector>
 #include <atomic>
 #include <mutex>
 #include "../../include/fastllm_hip.h"
@@ -298,6 +299,56 @@ struct flh_arena {
     size_t cap, used;
 };
 
+// A captured graph: the runtime's executable form, or, for a short chain of
+// kernels (a few layers' launches), the kernels themselves, launched one by
+// one.  The runtime's graph launch adds about 6 us on the device to every
+// replay (n kernels of 1.5 us: 7.7 + 1.53 n us) and 13 us or more on the host;
+// one by one they cost 2.26 us of host time each.  So the line: 1 / 4 / 8 / 12 /
+// 16 kernels of 2.6 us 2.9 / 10.8 / 21.7 / 32.6 / 43.4 us here, 15.8 / 17.5 /
+// 27.9 / 38.3 / 48.7 us as a graph; of 1.5 us 3.2 / 9.8 / 18.2 / 27.4 / 36.8 against
+// 16.6 / 13.9 / 20.0 / 26.1 / 32.2 (this library's shortest kernels take 1.8-2.2
+// us).  Longer chains and anything but a chain of kernels keep the runtime's form.
+namespace {
+struct graph_handle {
+    hipGraphExec_t exec = nullptr;
+    hipGraph_t graph = nullptr;
+    std::vector<hipKernelNodeParams> chain;                       // arguments owned by graph
+};
+constexpr size_t GRAPH_CHAIN_MAX = 16;
+
+// the nodes of g in order, if they are one chain of at most GRAPH_CHAIN_MAX kernels
+bool kernel_chain(hipGraph_t g, std::vector<hipKernelNodeParams> & out) {
+    size_t n = 0, one = 1;
+    hipGraphNode_t node;
+    if (hipGraphGetNodes(g, nullptr, &n) != hipSuccess || n == 0 || n > GRAPH_CHAIN_MAX) return false;
+    if (hipGraphGetRootNodes(g, nullptr, &one) != hipSuccess || one != 1) return false;
+    if (hipGraphGetRootNodes(g, &node, &one) != hipSuccess) return false;
+    out.clear();
+    for (size_t i = 0; i < n; ++i) {
+        hipGraphNodeType type;
+        hipKernelNodeParams k{};
+        if (hipGraphNodeGetType(node, &type) != hipSuccess || type != hipGraphNodeTypeKernel) return false;
+        if (hipGraphKernelNodeGetParams(node, &k) != hipSuccess || k.extra) return false;
+        // a kernel of a loaded module (not a host symbol) or a cooperative launch
+        // is the runtime's to replay
+        hipFuncAttributes fa;
+        if (hipFuncGetAttributes(&fa, k.func) != hipSuccess) {
+            (void)hipGetLastError();
+            return false;
+        }
+        hipKernelNodeAttrValue v{};
+        if (hipGraphKernelNodeGetAttribute(node, hipKernelNodeAttributeCooperative, &v) == hipSuccess && v.cooperative)
+            return false;
+        out.push_back(k);
+        size_t next = 0;
+        if (hipGraphNodeGetDependentNodes(node, nullptr, &next) != hipSuccess) return false;
+        if (next != (i + 1 < n ? 1u : 0u)) return false;
+        if (next && hipGraphNodeGetDependentNodes(node, &node, &next) != hipSuccess) return false;
+    }
+    return true;
+}
+}  // namespace
+
 extern "C" {
 
 const char * flh_last_error(void) { return g_err.c_str(); }
@@ -441,22 +492,40 @@ int flh_graph_capture_end(void * stream, void ** graph_exec) {
     hipGraph_t g = nullptr;
     // (with a null graph_exec the capture still ends, so the stream is usable)
     if (int rc = hip_check(hipStreamEndCapture((hipStream_t)stream, &g), "hipStreamEndCapture")) return rc;
-    hipGraphExec_t ge = nullptr;
     if (!graph_exec) {
         (void)hipGraphDestroy(g);
         return set_error(FLH_ERR_ARG, "null graph_exec");
     }
-    const int rc = hip_check(hipGraphInstantiate(&ge, g, nullptr, nullptr, 0), "hipGraphInstantiate");
-    (void)hipGraphDestroy(g);
-    if (rc) return rc;
-    *graph_exec = (void *)ge;
+    graph_handle * h = new graph_handle();
+    if (kernel_chain(g, h->chain)) {
+        h->graph = g;                                             // holds the arguments
+    } else {
+        const int rc = hip_check(hipGraphInstantiate(&h->exec, g, nullptr, nullptr, 0), "hipGraphInstantiate");
+        (void)hipGraphDestroy(g);
+        if (rc) {
+            delete h;
+            return rc;
+        }
+    }
+    *graph_exec = (void *)h;
     return FLH_OK;
 }
 int flh_graph_launch(void * ge, void * stream) {
-    return hip_check(hipGraphLaunch((hipGraphExec_t)ge, (hipStream_t)stream), "hipGraphLaunch");
+    const graph_handle * h = (const graph_handle *)ge;
+    if (!h) return set_error(FLH_ERR_ARG, "null graph");
+    if (h->exec) return hip_check(hipGraphLaunch(h->exec, (hipStream_t)stream), "hipGraphLaunch");
+    for (const hipKernelNodeParams & k : h->chain)
+        if (int rc = hip_check(hipLaunchKernel(k.func, k.gridDim, k.blockDim, k.kernelParams, k.sharedMemBytes,
+                                               (hipStream_t)stream), "graph kernel launch")) return rc;
+    return FLH_OK;
 }
 int flh_graph_destroy(void * ge) {
-    return ge ? hip_check(hipGraphExecDestroy((hipGraphExec_t)ge), "hipGraphExecDestroy") : FLH_OK;
+    graph_handle * h = (graph_handle *)ge;
+    if (!h) return FLH_OK;
+    const int rc = h->exec ? hip_check(hipGraphExecDestroy(h->exec), "hipGraphExecDestroy")
+                           : hip_check(hipGraphDestroy(h->graph), "hipGraphDestroy");
+    delete h;
+    return rc;
 }
 
 // ------------------------------------------------------------------- ops --
