@@ -160,8 +160,9 @@ static int dispatch_dot(int fmt, const DotArgs & a, int fast, uint32_t i8_mask, 
     if ((fmt == FLH_FMT_Q4_K || fmt == FLH_FMT_Q6_K) && ((i8k_mask >> fmt) & 1u))
         return launch_dot_i8k(fmt, a, s);
     if (fmt != FLH_FMT_F32 && ((i8_mask >> fmt) & 1u)) {
-        // Q8_0 / Q5_0: the matrix cores where they win (several columns, wide rows)
-        if (fmt == FLH_FMT_Q8_0 || fmt == FLH_FMT_Q5_0) {
+        // the 32-weight-block formats: the matrix cores where they win (several
+        // columns, wide rows)
+        if (fmt != FLH_FMT_Q4_K && fmt != FLH_FMT_Q6_K) {
             const int rc = launch_dot_cw(fmt, a, s);
             if (rc != FLH_ERR_UNSUPPORTED) return rc;
         }
@@ -190,7 +191,7 @@ static int dispatch_dot(int fmt, const DotArgs & a, int fast, uint32_t i8_mask, 
 }
 
 // Grouped expert dots of the 32-weight-block formats (Q8_0, Q5_0, IQ2_XXS,
-// IQ3_XXS x q8_1).  Q8_0 and Q5_0 of several tokens: the matrix cores, an
+// IQ3_XXS x q8_1).  Several tokens: the matrix cores, an
 // expert's weights streamed once for all of its pairs.  Otherwise the routed
 // superblock-per-lane launch, one workgroup row per (token, slot) pair (the
 // reference runs these per pair too, src/model/decoder.cpp:941-996).  Shapes its LDS plan cannot hold (rows of
@@ -205,6 +206,7 @@ static int launch_moe_b32(int fmt, const MoeArgs & a, hipStream_t s) {
     int rc = FLH_ERR_UNSUPPORTED;
     if (a.ntok > 1) rc = launch_moe_cw(fmt, a, s);
     if (rc == FLH_ERR_UNSUPPORTED) rc = launch_moe_sbl(fmt, a, s);
+    if (rc == FLH_ERR_UNSUPPORTED && a.ntok == 1) rc = launch_moe_cw(fmt, a, s);
     if (rc != FLH_ERR_UNSUPPORTED) return rc;
     for (uint32_t p = 0; p < a.ntok * a.top_k; ++p) {
         const uint32_t xi = a.x_per_slot ? p : p / a.top_k;
@@ -758,6 +760,7 @@ int flh_router_moe_dot(int fmt, const void * w, uint64_t estride, uint32_t rows,
         int rc = FLH_ERR_UNSUPPORTED;
         if (ntok > 1) rc = launch_moe_cw(fmt, f, s);
         if (rc == FLH_ERR_UNSUPPORTED && (ntok == 1 || !kf) && tune().sbl) rc = launch_moe_sbl(fmt, f, s);
+        if (rc == FLH_ERR_UNSUPPORTED && ntok == 1 && !kf) rc = launch_moe_cw(fmt, f, s);
         if (rc == FLH_ERR_UNSUPPORTED && kf) rc = launch_moe_kstream(fmt, f, s);
         if (rc != FLH_ERR_UNSUPPORTED) return rc;
     }

@@ -2,7 +2,7 @@
 // MoE experts) on the int8 matrix cores, one accumulator chain per wave.
 //
 // The reference folds a row's integer dots into four independent chains,
-// a[b & 3] over its blocks b (32 weights for Q8_0 / Q5_0, a superblock of 256
+// a[b & 3] over its blocks b (32 weights for Q8_0 / Q5_0 / IQ, a superblock of 256
 // for Q4_K / Q6_K), and adds (a0 + a1) + (a2 + a3) at the end
 // (src/runtime/quants.h:438-594).  Here a workgroup of four waves owns 16 rows
 // at a time and wave k runs chain k of all of them, so a chain is a register
@@ -35,6 +35,15 @@
 // free of bank conflicts; 8 bytes of every block per lane (a plain A operand)
 // took 742 LDS cycles per chunk instead of about 140.
 //
+// IQ2_XXS / IQ3_XXS: 1024 columns a chunk, 8 blocks per wave in two halves that
+// run as Q8_0's; a lane expands its block from the codebook and a table of sign
+// masks in LDS (the consumers copy both in while the first chunks fly).  Rows lie
+// at 2-byte offsets, so a row of any number of superblocks is taken from the
+// 16-byte boundary below, as Q6_K's.  Bound by the DMA instructions: 28672x4096
+// IQ2_XXS with 4 / 8 / 16 columns 20.9 / 29 / 44 us, 27.6 / 41 / 82 one lane per
+// half superblock; 3840x3840 with 16 columns 44 -> 10.2 (register kernel before);
+// six of 64 experts of 1536x2560, 3 tokens: 237 -> 60 us a layer.
+//
 // Bound by the DMA: with 4 columns 28672x4096 Q8_0 takes 25.9 us (4.8 TB/s) where
 // streaming the chunks alone takes 25.1; with 16 columns the activations are as
 // many bytes again (38 us).
@@ -52,29 +61,34 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 constexpr int CW_AUX = 2;
 
 // UB: weight bytes per 256 columns; CU: 256-column units per chunk; WSEG:
-// 16-byte segments of a row's chunk (Q6_K: 840 bytes from a 16-byte boundary
-// up to 14 bytes below); UA: appendix bytes per unit; ASEG: segments per
+// 16-byte segments of a row's chunk (Q6_K, IQ2_XXS, IQ3_XXS: its bytes from a
+// 16-byte boundary up to 14 bytes below); UA: appendix bytes per unit; ASEG: segments per
 // column of a chunk's activations.
 template <int FMT> struct CW;
 template <> struct CW<FMT_Q8_0> { static constexpr uint32_t UB = 272, CU = 2, WSEG = 34, UA = 288, ASEG = 36; };
 template <> struct CW<FMT_Q5_0> { static constexpr uint32_t UB = 176, CU = 2, WSEG = 22, UA = 288, ASEG = 36; };
 template <> struct CW<FMT_Q4_K> { static constexpr uint32_t UB = 144, CU = 4, WSEG = 36, UA = 292, ASEG = 73; };
 template <> struct CW<FMT_Q6_K> { static constexpr uint32_t UB = 210, CU = 4, WSEG = 54, UA = 292, ASEG = 73; };
+template <> struct CW<FMT_IQ2_XXS> { static constexpr uint32_t UB = 66, CU = 4, WSEG = 18, UA = 288, ASEG = 72; };
+template <> struct CW<FMT_IQ3_XXS> { static constexpr uint32_t UB = 98, CU = 4, WSEG = 26, UA = 288, ASEG = 72; };
+// the codebook formats; the formats whose superblocks are 2-byte aligned
+__host__ __device__ constexpr bool cw_iq(int fmt) { return fmt == FMT_IQ2_XXS || fmt == FMT_IQ3_XXS; }
+__host__ __device__ constexpr bool cw_gran(int fmt) { return fmt == FMT_Q6_K || cw_iq(fmt); }
 
 // DMA instructions of a chunk: the rows' segments, the columns' segments, and
-// (32-weight formats) the 16 blocks' {d, s} words of every column again, as a
+// (32-weight blocks) the blocks' {d, s} words of every column again, as a
 // table [block][NC] whose four words a lane reads at once.
 template <int FMT, int NC> struct CwPlan {
     static constexpr bool KF = FMT == FMT_Q4_K || FMT == FMT_Q6_K;
     static constexpr uint32_t NW = (16 * CW<FMT>::WSEG + 63) / 64, NA = (NC * CW<FMT>::ASEG + 63) / 64;
-    static constexpr uint32_t NX = KF ? 0 : NC / 4, NT = NW + NA + NX;
+    static constexpr uint32_t NX = KF ? 0 : NC * CW<FMT>::CU / 8, NT = NW + NA + NX;
     static constexpr uint32_t XOFF = (NW + NA) * 1024, STG = XOFF + NX * 256;
 };
 constexpr uint32_t CW_WAVES = 5;                                  // four consumers and the producer
 constexpr uint32_t CW_ZERO = 320;                                 // zero bytes that off-diagonal lanes read
-// LDS: [D][STG] ring | [4][16][16] sums | zeros
+// LDS: [D][STG] ring | [4][16][16] sums | zeros | codebook (2 KiB), sign masks (1 KiB)
 template <int FMT, int NC> __host__ __device__ constexpr size_t cw_smem(int D) {
-    return (size_t)D * CwPlan<FMT, NC>::STG + 4096 + CW_ZERO;
+    return (size_t)D * CwPlan<FMT, NC>::STG + 4096 + CW_ZERO + (cw_iq(FMT) ? 3072 : 0);
 }
 
 // Activation column p starts xoff(p) bytes after base() (the launcher bounds
@@ -127,6 +141,9 @@ __device__ __forceinline__ float cw_hmul(uint32_t a, uint32_t b, float nz) {
 // dwords at an LDS offset
 typedef const __attribute__((address_space(3))) uint32_t * lds32;
 typedef const __attribute__((address_space(3))) u32x2 * lds64;
+typedef const __attribute__((address_space(3))) uint16_t * lds16;
+typedef __attribute__((address_space(3))) uint32_t * lds32w;
+typedef __attribute__((address_space(3))) u32x2 * lds64w;
 __device__ __forceinline__ lds32 lp32(uint32_t off) { return (lds32)(uintptr_t)off; }
 __device__ __forceinline__ u32x2 lp64(uint32_t off) { return *(lds64)(uintptr_t)off; }
 
@@ -161,7 +178,7 @@ __device__ __forceinline__ void cw_produce(const uint8_t * __restrict__ w, uint3
     uint32_t vo[NT];
     auto w_off = [&](uint32_t q, uint32_t nv, uint32_t lim) -> uint32_t {
         const uint32_t s = min(64 * q + lane, 16 * P::WSEG - 1);
-        return min(s / P::WSEG, nv) * RB + (FMT == FMT_Q6_K ? 0u : min(16 * (s % P::WSEG), lim));
+        return min(s / P::WSEG, nv) * RB + (cw_gran(FMT) ? 0u : min(16 * (s % P::WSEG), lim));
     };
     auto a_off = [&](uint32_t q, uint32_t lim) -> uint32_t {
         const uint32_t s = min(64 * (q - NW) + lane, NC * P::ASEG - 1), n = s / P::ASEG;
@@ -172,7 +189,7 @@ __device__ __forceinline__ void cw_produce(const uint8_t * __restrict__ w, uint3
         return C.xoff(n < nx ? n : 0) + 36 * min(e / NC, lim);
     };
 #pragma unroll
-    for (uint32_t q = NW; q < NT; ++q) vo[q] = q < NW + NA ? a_off(q, ALIM) : x_off(q, 15);
+    for (uint32_t q = NW; q < NT; ++q) vo[q] = q < NW + NA ? a_off(q, ALIM) : x_off(q, 8 * P::CU - 1);
     uint32_t qt = 0, qc = 0, qslot = 0;                           // next chunk to issue
     auto issue_next = [&]() __attribute__((always_inline)) {
         if (qt >= ntile) return;
@@ -184,13 +201,13 @@ __device__ __forceinline__ void cw_produce(const uint8_t * __restrict__ w, uint3
         uint8_t * stage = sm + (size_t)qslot * STG;
         const uint8_t * wb = w + (size_t)row0 * RB + (size_t)qc * CB;
         const uint8_t * xb = x0 + (size_t)qc * CA;
-        if (qc + 1 < nch || lastu == P::CU || FMT == FMT_Q6_K) {
-            const uint32_t sh = (uint32_t)(uintptr_t)wb & 15u;    // Q6_K: the chunk's offset in its granule
-            const bool part = qc + 1 == nch && lastu < P::CU;     // (Q6_K only)
+        if (qc + 1 < nch || lastu == P::CU || cw_gran(FMT)) {
+            const uint32_t sh = (uint32_t)(uintptr_t)wb & 15u;    // the chunk's offset in its granule
+            const bool part = qc + 1 == nch && lastu < P::CU;     // (these formats only)
             const uint32_t wbytes = (part ? lastu : P::CU) * P::UB;
 #pragma unroll
             for (uint32_t q = 0; q < NW; ++q) {
-                if constexpr (FMT == FMT_Q6_K) {
+                if constexpr (cw_gran(FMT)) {
                     // segments from the boundary below the row's chunk to the
                     // granule of its last byte
                     const uint32_t s = min(64 * q + lane, 16 * P::WSEG - 1) % P::WSEG;
@@ -206,7 +223,8 @@ __device__ __forceinline__ void cw_produce(const uint8_t * __restrict__ w, uint3
                                                  LPTR(stage + 1024 * q), 16, 0, 0);
 #pragma unroll
             for (uint32_t q = NW + NA; q < NT; ++q)
-                __builtin_amdgcn_global_load_lds(GPTR(xb + vo[q]), LPTR(stage + L::XOFF + 256 * (q - NW - NA)), 4, 0, 0);
+                __builtin_amdgcn_global_load_lds(GPTR(xb + (part ? x_off(q, 8 * lastu - 1) : vo[q])),
+                                                 LPTR(stage + L::XOFF + 256 * (q - NW - NA)), 4, 0, 0);
         } else {                                                  // a partial last chunk: no read past the row or column
 #pragma unroll
             for (uint32_t q = 0; q < NW; ++q)
@@ -263,6 +281,16 @@ __device__ __forceinline__ void cw_consume(const uint8_t * __restrict__ w, uint3
     asm volatile("" : "+v"(nz));                                  // kept as a register
     const uint32_t p = tid >> 4;                                  // this thread's (column, row) of the sums
     uint32_t slot = 0;
+    [[maybe_unused]] const uint32_t grid = zr + CW_ZERO;
+    if constexpr (cw_iq(FMT)) {                                   // (read after the first chunk's barrier)
+        if constexpr (FMT == FMT_IQ2_XXS) {
+            *(lds64w)(uintptr_t)(grid + 8 * tid) = u32x2{(uint32_t)k_iq2_grid[tid], (uint32_t)(k_iq2_grid[tid] >> 32)};
+        } else {
+            *(lds32w)(uintptr_t)(grid + 4 * tid) = k_iq3_grid[tid];
+        }
+        const uint32_t sg = iq_sign8(tid & 127u);
+        *(lds64w)(uintptr_t)(grid + 2048 + 8 * (tid & 127u)) = u32x2{iq_neg4(sg), iq_neg4(sg >> 4)};
+    }
     for (uint32_t t = 0; t < ntile; ++t) {
         const uint32_t row = rbeg + 16 * t + (tid & 15);
         const bool mine = p < nx && row < rend;
@@ -277,7 +305,73 @@ __device__ __forceinline__ void cw_consume(const uint8_t * __restrict__ w, uint3
             const uint32_t xs = st + 1024 * L::NW, xt = st + L::XOFF;   // the columns, the table
             slot = slot + 1 == (uint32_t)D ? 0 : slot + 1;
             const uint32_t units = c + 1 == nch ? lastu : P::CU;
-            if constexpr (!KF) {
+            if constexpr (cw_iq(FMT)) {
+                // lane (r, j): blocks b = 16 h + 4 j + k of row r, group 4 (j & 1) + k
+                // of superblock 2 h + j / 2; the row's chunk starts sh bytes into its window
+                const uint32_t wrow = min(rbeg + 16 * t + r, rend - 1);
+                const uint32_t sh = ((uint32_t)(uintptr_t)w + wrow * RB + c * CB) & 15u;
+                const bool diag = (r >> 2) == j;
+#pragma unroll
+                for (uint32_t h = 0; h < 2; ++h) {
+                    if (2 * h >= units) break;
+                    const uint32_t g = 4 * (j & 1) + k, sb = st + r * WROW + sh + P::UB * (2 * h + (j >> 1));
+                    const uint32_t hd = *(lds16)(uintptr_t)sb;
+                    // w1 and the grid indices, from aligned dwords
+                    const uint32_t ga = sb + 2 + 8 * g, s2 = ga & 2u;
+                    const lds32 gp = lp32(ga - s2);
+                    const uint32_t i0 = alignb(gp[1], gp[0], s2);
+                    uint32_t w1 = alignb(gp[2], gp[1], s2), E[8];
+                    if constexpr (FMT == FMT_IQ2_XXS) {           // an 8-byte entry per run
+#pragma unroll
+                        for (int l = 0; l < 4; ++l) {
+                            const u32x2 e = lp64(grid + 8 * ((i0 >> (8 * l)) & 0xFFu));
+                            E[2 * l] = e.x;
+                            E[2 * l + 1] = e.y;
+                        }
+                    } else {                                      // two 4-byte entries per run
+                        const uint32_t i1 = w1;
+                        const lds32 wp = lp32(ga - s2 + 64 - 4 * g);
+                        w1 = alignb(wp[1], wp[0], s2);
+#pragma unroll
+                        for (int l = 0; l < 8; ++l)
+                            E[l] = *lp32(grid + 4 * (((l < 4 ? i0 : i1) >> (8 * (l & 3))) & 0xFFu));
+                    }
+#pragma unroll
+                    for (int l = 0; l < 4; ++l) {
+                        const u32x2 n = lp64(grid + 2048 + 8 * ((w1 >> (7 * l)) & 127u));
+                        E[2 * l] = iq_apply(E[2 * l], n.x);
+                        E[2 * l + 1] = iq_apply(E[2 * l + 1], n.y);
+                    }
+                    const float db = iq_db(FMT, h2f(hd), w1);
+                    const v4i b0 = {(int)E[0], (int)E[1], (int)E[2], (int)E[3]}, b1 = {(int)E[4], (int)E[5], (int)E[6], (int)E[7]};
+                    const uint32_t b = 16 * h + 4 * j + k;
+#pragma unroll
+                    for (int gr = 0; gr < NG; ++gr) {
+                        // A as for Q8_0 below
+                        const lds32 ap = lp32(diag ? xs + (4 * gr + (r & 3)) * AROW + 36 * b + 4 : zr);
+                        const v4i a0 = {(int)ap[0], (int)ap[1], (int)ap[2], (int)ap[3]};
+                        const v4i a1 = {(int)ap[4], (int)ap[5], (int)ap[6], (int)ap[7]};
+                        const u32x4a dx = *(const __attribute__((address_space(3))) u32x4a *)(uintptr_t)(
+                            xt + (b * NC + 4 * gr) * 4);
+                        v4i d = __builtin_amdgcn_mfma_i32_16x16x64_i8(a0, b0, v4i{0, 0, 0, 0}, 0, 0, 0);
+                        d = __builtin_amdgcn_mfma_i32_16x16x64_i8(a1, b1, d, 0, 0, 0);
+                        uint32_t m[4], f[4];
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            m[i] = __float_as_uint(db * h2f(dx[i] & 0xFFFFu));
+                            f[i] = (uint32_t)d[i];
+                        }
+                        cw_transpose(m);                          // lane row j: column 4 gr + j, blocks t = 0..3
+                        cw_transpose(f);
+                        acc[gr] = fmaf(__uint_as_float(m[0]), (float)(int)f[0], acc[gr]);
+                        acc[gr] = fmaf(__uint_as_float(m[1]), (float)(int)f[1], acc[gr]);
+                        if (units > 2 * h + 1) {                  // (blocks 2 and 3 lie in the second superblock)
+                            acc[gr] = fmaf(__uint_as_float(m[2]), (float)(int)f[2], acc[gr]);
+                            acc[gr] = fmaf(__uint_as_float(m[3]), (float)(int)f[3], acc[gr]);
+                        }
+                    }
+                }
+            } else if constexpr (!KF) {
                 // lane (r, j): block b = 4 j + k of row r
                 auto chain = [&](auto kc) __attribute__((always_inline)) {
                     constexpr int K = decltype(kc)::value, BB = FMT == FMT_Q8_0 ? 34 : 22;
@@ -538,9 +632,9 @@ static bool cw_takes(int fmt, const void * w, uint64_t estride, const void * x, 
     if (cols == 0 || (cols & 255) || ((uintptr_t)x & 15) || (xstride & 3)) return false;
     // 32-bit lane offsets
     if ((uint64_t)ncol * xstride * 4 + x_alloc_bytes(cols) >= (1ull << 32) || 16ull * cols * 2 >= (1ull << 32)) return false;
-    // Q6_K rows are placed from their own 16-byte boundaries; the others' rows
+    // Q6_K and IQ rows are placed from their own 16-byte boundaries; the others' rows
     // and pieces are whole 16-byte segments of an aligned matrix
-    const uintptr_t al = fmt == FMT_Q6_K ? 1 : 15;
+    const uintptr_t al = cw_gran(fmt) ? 1 : 15;
     return !((uintptr_t)w & al) && !(estride & al);
 }
 
@@ -599,10 +693,21 @@ template <int FMT> static int cw_launch(const DotArgs & a, hipStream_t s) {
 //    than its one pass per lane group holds well, Q8_0 4096x14336 14.7 / 18.3,
 //    8192x8192 14.7 / 17.0, Q5_0 27648x5120 22.6 / 32.8; not 14336x4096 15.2 / 13.4,
 //    2048x5632 7.6 / 6.3.
+//  * IQ2_XXS and IQ3_XXS against k_dot_sbl_nx (rows of up to 8192 columns, a
+//    multiple of 2048), k_dot_sbl (one column) and the register kernel: IQ2_XXS
+//    14336x4096 with 2 / 4 / 8 / 16 columns 13.8 / 12.5, 13.7 / 14.8, 18.2 / 21.5,
+//    26.7 / 42.5; 28672x4096 with 2 20.9 / 22.8; 4096x14336 with 2 / 8 16.2 / 26.8,
+//    20.4 / 61.6; IQ3_XXS 14336x4096 with 2 / 4 16.2 / 14.6, 16.1 / 16.9.  Rows
+//    that are no multiple of 2048 columns, 3840x3840 with 1 / 2 / 16: 6.5 / 7.7,
+//    6.5 / 8.7, 10.2 / 44; one column of few rows, 1024x2816: 5.4 / 5.1.
 static bool cw_wins(int fmt, uint32_t rows, uint32_t cols, uint32_t nx) {
     const uint32_t T = (rows + 15) / 16, cus = (uint32_t)num_cus();
     if (fmt == FMT_Q4_K) return nx <= 4 || (nx <= 8 ? rows <= 16384 : T <= cus || cols > 4096);
     if (fmt == FMT_Q6_K) return nx > 2 || cols > 8192;
+    if (cw_iq(fmt)) {
+        if (nx == 1) return cols > 16128 || ((cols & 2047) && rows >= 2048);
+        return nx > 2 || cols > 8192 || (cols & 2047) || rows > 16384;
+    }
     if (nx == 1) return cols > 4096 && T >= cus;
     if (nx <= 4 && 4 * T <= cus && cols > 2048) return false;
     return nx > 2 || fmt == FMT_Q5_0 || cols > 4096;
@@ -621,6 +726,8 @@ int launch_dot_cw(int fmt, const DotArgs & a, hipStream_t s) {
         case FMT_Q5_0: return cw_launch<FMT_Q5_0>(a, s);
         case FMT_Q4_K: return cw_launch<FMT_Q4_K>(a, s);
         case FMT_Q6_K: return cw_launch<FMT_Q6_K>(a, s);
+        case FMT_IQ2_XXS: return cw_launch<FMT_IQ2_XXS>(a, s);
+        case FMT_IQ3_XXS: return cw_launch<FMT_IQ3_XXS>(a, s);
         default: return FLH_ERR_UNSUPPORTED;
     }
 }
@@ -653,6 +760,8 @@ int launch_moe_cw(int fmt, const MoeArgs & a, hipStream_t s) {
         case FMT_Q5_0: return cw_moe<FMT_Q5_0>(a, s);
         case FMT_Q4_K: return cw_moe<FMT_Q4_K>(a, s);
         case FMT_Q6_K: return cw_moe<FMT_Q6_K>(a, s);
+        case FMT_IQ2_XXS: return cw_moe<FMT_IQ2_XXS>(a, s);
+        case FMT_IQ3_XXS: return cw_moe<FMT_IQ3_XXS>(a, s);
         default: return FLH_ERR_UNSUPPORTED;
     }
 }
