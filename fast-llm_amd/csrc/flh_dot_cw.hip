@@ -25,12 +25,16 @@
 // SIMD where a matrix has one tile per CU): Q8_0 4096x14336 with 4 columns
 // 21.5 us, 15.0 with the producer; streaming alone takes 13.8.
 //
-// The A operand is block-diagonal: row n holds column n % 4 of a group of 4
-// (Q6_K: n % 8 of 8) on the k-slice n / 4 (the slices of sub-block n / 8) only,
-// so each 16-lane row j of the result holds the dots of that slice's own block:
-// Q8_0 / Q5_0 the j-th block of the chain in the chunk (a 4 x 4 transpose by
-// permlane swaps then gives lane row j column j's four blocks in order), Q4_K
-// sub-blocks 2 j and 2 j + 1 (summed over the rows by swaps, integers, exact).
+// The A operand is block-diagonal: row n holds column n / 4 of a group of 4
+// on k-slice n % 4 only (Q6_K: column n / 2 of 8 on the slices of sub-block n %
+// 2), so 16-lane row j of the result holds column j's dots with the four blocks
+// of lane rows 0-3: Q8_0 / Q5_0 the chain's four blocks in the chunk, in order
+// (their scales are gathered from the lane rows once per chunk, for all
+// columns), Q4_K the superblock's sub-blocks, scaled and added as integers.  With
+// column n % 4 on slice n / 4 (each lane row its own block's dots) results and
+// scales had to be transposed per group, eight lane-row swaps: Q8_0 28672x4096
+// with 16 columns 34.6 -> 32.8 us, IQ2_XXS 4096x14336 29.0 -> 25.4, Q4_K 16.4 ->
+// 14.9, Q6_K vocabulary 128256x4096 with 5 / 16 columns 89.9 -> 88.9, 120 -> 114.
 // A lane reads one block's contiguous bytes, which for the 32-weight formats is
 // free of bank conflicts; 8 bytes of every block per lane (a plain A operand)
 // took 742 LDS cycles per chunk instead of about 140.
@@ -39,14 +43,15 @@
 // run as Q8_0's; a lane expands its block from the codebook and a table of sign
 // masks in LDS (the consumers copy both in while the first chunks fly).  Rows lie
 // at 2-byte offsets, so a row of any number of superblocks is taken from the
-// 16-byte boundary below, as Q6_K's.  Bound by the DMA instructions: 28672x4096
-// IQ2_XXS with 4 / 8 / 16 columns 20.9 / 29 / 44 us, 27.6 / 41 / 82 one lane per
-// half superblock; 3840x3840 with 16 columns 44 -> 10.2 (register kernel before);
+// 16-byte boundary below, as Q6_K's.  Bound by the expansion and the folds:
+// 28672x4096 IQ2_XXS with 4 / 8 / 16 columns 20.6 / 28.6 / 42 us, 27.6 / 41 / 82 one
+// lane per half superblock; 3840x3840 with 16 columns 44 -> 10.2 (register kernel before);
 // six of 64 experts of 1536x2560, 3 tokens: 237 -> 60 us a layer.
 //
-// Bound by the DMA: with 4 columns 28672x4096 Q8_0 takes 25.9 us (4.8 TB/s) where
-// streaming the chunks alone takes 25.1; with 16 columns the activations are as
-// many bytes again (38 us).
+// Bound by the weight stream with few columns (28672x4096 Q8_0 with 4 24.2 us, 5.2
+// TB/s; streaming the chunks alone takes 25.1 where the whole kernel took 25.9), by
+// the consumers beyond: with 16 columns 32.8 us, and staging fewer activation
+// bytes (32-row tiles, or only the columns that are there) changes nothing.
 #include "flh_kstream.h"
 #include "flh_internal.h"
 #include "flh_status.h"
@@ -77,7 +82,7 @@ __host__ __device__ constexpr bool cw_gran(int fmt) { return fmt == FMT_Q6_K || 
 
 // DMA instructions of a chunk: the rows' segments, the columns' segments, and
 // (32-weight blocks) the blocks' {d, s} words of every column again, as a
-// table [block][NC] whose four words a lane reads at once.
+// table [column][16 blocks][chain][4] whose four words a lane reads at once.
 template <int FMT, int NC> struct CwPlan {
     static constexpr bool KF = FMT == FMT_Q4_K || FMT == FMT_Q6_K;
     static constexpr uint32_t NW = (16 * CW<FMT>::WSEG + 63) / 64, NA = (NC * CW<FMT>::ASEG + 63) / 64;
@@ -112,26 +117,22 @@ struct CwColsMoe {
     __device__ float * y(uint32_t p) const { return y0 + (size_t)lds_ld32(&yi[p]) * ys; }
 };
 
-// Transpose over the four 16-lane rows: row j leaves with v[t] = the v[j] of row t.
-__device__ __forceinline__ void cw_transpose(uint32_t (&v)[4]) {
-    const auto a = __builtin_amdgcn_permlane32_swap(v[0], v[2], false, false);
-    const auto b = __builtin_amdgcn_permlane32_swap(v[1], v[3], false, false);
-    const auto c = __builtin_amdgcn_permlane16_swap(a[0], b[0], false, false);
-    const auto d = __builtin_amdgcn_permlane16_swap(a[1], b[1], false, false);
-    v[0] = c[0]; v[1] = c[1]; v[2] = d[0]; v[3] = d[1];
-}
-// Sum over the four 16-lane rows, transposed: row j gets the sum of p[j].
-// Integer adds: exact in any order.
-__device__ __forceinline__ int cw_rowsum(const int (&p)[4]) {
-    const auto a = __builtin_amdgcn_permlane32_swap((uint32_t)p[0], (uint32_t)p[2], false, false);
-    const auto b = __builtin_amdgcn_permlane32_swap((uint32_t)p[1], (uint32_t)p[3], false, false);
-    const auto c = __builtin_amdgcn_permlane16_swap(a[0] + a[1], b[0] + b[1], false, false);
-    return (int)(c[0] + c[1]);
+// All four 16-lane rows' values: g[t] = the v of lane row t.
+__device__ __forceinline__ void cw_gather(uint32_t v, uint32_t (&g)[4]) {
+    const auto a = __builtin_amdgcn_permlane32_swap(v, v, false, false);   // rows 0 1 0 1, 2 3 2 3
+    const auto b = __builtin_amdgcn_permlane16_swap(a[0], a[0], false, false);
+    const auto c = __builtin_amdgcn_permlane16_swap(a[1], a[1], false, false);
+    g[0] = b[0]; g[1] = b[1]; g[2] = c[0]; g[3] = c[1];
 }
 // d_w * d_x of two halves (the low or the high one of a, the low one of b) as
 // binary32: exact (22 significant bits), so the same as the product of the
 // widened values; as a mixed-precision fma with nz = -0.0 (kept opaque) it is
 // one instruction instead of two conversions and a multiplication.
+// (cw_fmul: of a binary32 and a half, rounded once)
+__device__ __forceinline__ float cw_fmul(uint32_t a, uint32_t b, float nz) {
+    typedef _Float16 h2v __attribute__((ext_vector_type(2)));
+    return __builtin_fmaf(__uint_as_float(a), (float)__builtin_bit_cast(h2v, b).x, nz);
+}
 template <bool HI>
 __device__ __forceinline__ float cw_hmul(uint32_t a, uint32_t b, float nz) {
     typedef _Float16 h2v __attribute__((ext_vector_type(2)));
@@ -157,6 +158,15 @@ __device__ __forceinline__ void cw_wait(uint32_t behind) {
     if constexpr (B > 0) cw_wait<B - 1, N>(behind);
 }
 
+// The thread's index, opaque: a kernel that holds several forms of the body
+// must not compute all their addresses up front (230 registers, one workgroup
+// per CU).
+__device__ __forceinline__ uint32_t cw_tid() {
+    uint32_t t = threadIdx.x;
+    asm volatile("" : "+v"(t));
+    return t;
+}
+
 // The producer wave: streams the chunks of rows [rbeg, rend), D - 1 ahead.
 // vo: per instruction the lane's byte offset from the chunk's start in the
 // tile's first row (rows), or in column 0's appendix (columns, table); the
@@ -170,33 +180,33 @@ __device__ __forceinline__ void cw_produce(const uint8_t * __restrict__ w, uint3
     constexpr uint32_t NT = L::NT, STG = L::STG, NW = L::NW, NA = L::NA;
     constexpr uint32_t CB = P::CU * P::UB, CA = P::CU * P::UA;
     static_assert((D - 2) * (int)NT <= 60, "vmcnt counts to 63");
-    const uint32_t lane = threadIdx.x & 63;
+    const uint32_t lane = cw_tid() & 63;
     const uint32_t nsb = cols >> 8, nch = (nsb + P::CU - 1) / P::CU, lastu = nsb - (nch - 1) * P::CU;
     const uint32_t RB = nsb * P::UB, ntile = (rend - rbeg + 15) >> 4, total = ntile * nch;
     const uint8_t * const x0 = reinterpret_cast<const uint8_t *>(C.base()) + (KF ? xqk_off(cols) : xq_off(cols));
     constexpr uint32_t ALIM = 16 * P::ASEG - 16;                  // a column's last segment
     uint32_t vo[NT];
-    auto w_off = [&](uint32_t q, uint32_t nv, uint32_t lim) -> uint32_t {
-        const uint32_t s = min(64 * q + lane, 16 * P::WSEG - 1);
+    auto w_off = [&](uint32_t ln, uint32_t q, uint32_t nv, uint32_t lim) -> uint32_t {
+        const uint32_t s = min(64 * q + ln, 16 * P::WSEG - 1);
         return min(s / P::WSEG, nv) * RB + (cw_gran(FMT) ? 0u : min(16 * (s % P::WSEG), lim));
     };
-    auto a_off = [&](uint32_t q, uint32_t lim) -> uint32_t {
-        const uint32_t s = min(64 * (q - NW) + lane, NC * P::ASEG - 1), n = s / P::ASEG;
+    auto a_off = [&](uint32_t ln, uint32_t q, uint32_t lim) -> uint32_t {
+        const uint32_t s = min(64 * (q - NW) + ln, NC * P::ASEG - 1), n = s / P::ASEG;
         return C.xoff(n < nx ? n : 0) + min(16 * (s % P::ASEG), lim);
     };
-    auto x_off = [&](uint32_t q, uint32_t lim) -> uint32_t {
-        const uint32_t e = 64 * (q - NW - NA) + lane, n = e % NC;
-        return C.xoff(n < nx ? n : 0) + 36 * min(e / NC, lim);
+    auto x_off = [&](uint32_t ln, uint32_t q, uint32_t lim) -> uint32_t {
+        const uint32_t e = 64 * (q - NW - NA) + ln, n = e / (8 * P::CU), i = e % (8 * P::CU);
+        return C.xoff(n < nx ? n : 0) + 36 * min((i & ~15u) + 4 * (i & 3) + ((i >> 2) & 3), lim);
     };
 #pragma unroll
-    for (uint32_t q = NW; q < NT; ++q) vo[q] = q < NW + NA ? a_off(q, ALIM) : x_off(q, 8 * P::CU - 1);
+    for (uint32_t q = NW; q < NT; ++q) vo[q] = q < NW + NA ? a_off(lane, q, ALIM) : x_off(lane, q, 8 * P::CU - 1);
     uint32_t qt = 0, qc = 0, qslot = 0;                           // next chunk to issue
     auto issue_next = [&]() __attribute__((always_inline)) {
         if (qt >= ntile) return;
         const uint32_t row0 = rbeg + 16 * qt, nv = min(15u, rend - 1 - row0);   // nv: last row of the tile
         if (qc == 0 && (qt == 0 || nv < 15)) {                    // the offsets differ only in a partial tile
 #pragma unroll
-            for (uint32_t q = 0; q < NW; ++q) vo[q] = w_off(q, nv, 0xFFFFu);
+            for (uint32_t q = 0; q < NW; ++q) vo[q] = w_off(lane, q, nv, 0xFFFFu);
         }
         uint8_t * stage = sm + (size_t)qslot * STG;
         const uint8_t * wb = w + (size_t)row0 * RB + (size_t)qc * CB;
@@ -205,6 +215,8 @@ __device__ __forceinline__ void cw_produce(const uint8_t * __restrict__ w, uint3
             const uint32_t sh = (uint32_t)(uintptr_t)wb & 15u;    // the chunk's offset in its granule
             const bool part = qc + 1 == nch && lastu < P::CU;     // (these formats only)
             const uint32_t wbytes = (part ? lastu : P::CU) * P::UB;
+            uint32_t ln = lane;
+            asm volatile("" : "+v"(ln));                          // (see below)
 #pragma unroll
             for (uint32_t q = 0; q < NW; ++q) {
                 if constexpr (cw_gran(FMT)) {
@@ -219,24 +231,30 @@ __device__ __forceinline__ void cw_produce(const uint8_t * __restrict__ w, uint3
             }
 #pragma unroll
             for (uint32_t q = NW; q < NW + NA; ++q)
-                __builtin_amdgcn_global_load_lds(GPTR(xb + (part ? a_off(q, (lastu * P::UA - 1) & ~15u) : vo[q])),
+                __builtin_amdgcn_global_load_lds(GPTR(xb + (part ? a_off(ln, q, (lastu * P::UA - 1) & ~15u) : vo[q])),
                                                  LPTR(stage + 1024 * q), 16, 0, 0);
 #pragma unroll
             for (uint32_t q = NW + NA; q < NT; ++q)
-                __builtin_amdgcn_global_load_lds(GPTR(xb + (part ? x_off(q, 8 * lastu - 1) : vo[q])),
+                __builtin_amdgcn_global_load_lds(GPTR(xb + (part ? x_off(ln, q, 8 * lastu - 1) : vo[q])),
                                                  LPTR(stage + L::XOFF + 256 * (q - NW - NA)), 4, 0, 0);
         } else {                                                  // a partial last chunk: no read past the row or column
+            // its offsets are made anew (the opaque lane): kept next to the whole
+            // chunk's they took the producer over 128 registers, and waves that
+            // need more leave a CU one workgroup (Q4_K 28672x4096 with 16 columns
+            // 31.7 us, 24.9 within 128)
+            uint32_t ln = lane;
+            asm volatile("" : "+v"(ln));
 #pragma unroll
             for (uint32_t q = 0; q < NW; ++q)
-                __builtin_amdgcn_global_load_lds(GPTR(wb + w_off(q, nv, lastu * P::UB - 16)), LPTR(stage + 1024 * q), 16, 0,
+                __builtin_amdgcn_global_load_lds(GPTR(wb + w_off(ln, q, nv, lastu * P::UB - 16)), LPTR(stage + 1024 * q), 16, 0,
                                                  CW_AUX);
 #pragma unroll
             for (uint32_t q = NW; q < NW + NA; ++q)
-                __builtin_amdgcn_global_load_lds(GPTR(xb + a_off(q, (lastu * P::UA - 1) & ~15u)), LPTR(stage + 1024 * q), 16,
+                __builtin_amdgcn_global_load_lds(GPTR(xb + a_off(ln, q, (lastu * P::UA - 1) & ~15u)), LPTR(stage + 1024 * q), 16,
                                                  0, 0);
 #pragma unroll
             for (uint32_t q = NW + NA; q < NT; ++q)
-                __builtin_amdgcn_global_load_lds(GPTR(xb + x_off(q, 8 * lastu - 1)),
+                __builtin_amdgcn_global_load_lds(GPTR(xb + x_off(ln, q, 8 * lastu - 1)),
                                                  LPTR(stage + L::XOFF + 256 * (q - NW - NA)), 4, 0, 0);
         }
         qslot = qslot + 1 == (uint32_t)D ? 0 : qslot + 1;
@@ -262,7 +280,7 @@ __device__ __forceinline__ void cw_consume(const uint8_t * __restrict__ w, uint3
     using L = CwPlan<FMT, NC>;
     constexpr bool KF = L::KF;
     constexpr uint32_t STG = L::STG, WROW = 16 * P::WSEG, AROW = 16 * P::ASEG, CB = P::CU * P::UB;
-    const uint32_t tid = threadIdx.x, lane = tid & 63;
+    const uint32_t tid = cw_tid(), lane = tid & 63;
     const uint32_t k = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t r = lane & 15, j = lane >> 4;
     const uint32_t nsb = cols >> 8, nch = (nsb + P::CU - 1) / P::CU, lastu = nsb - (nch - 1) * P::CU;
@@ -275,7 +293,7 @@ __device__ __forceinline__ void cw_consume(const uint8_t * __restrict__ w, uint3
     // the lane's i-th output column
     auto col_of = [&](int i) -> uint32_t {
         if constexpr (FMT != FMT_Q6_K) return 4 * i + j;
-        else return 8 * (i >> 1) + 4 * (j & 1) + 2 * (j >> 1) + (i & 1);
+        else return 8 * (i >> 1) + 2 * j + (i & 1);
     };
     [[maybe_unused]] float nz = -0.0f;
     asm volatile("" : "+v"(nz));                                  // kept as a register
@@ -310,7 +328,7 @@ __device__ __forceinline__ void cw_consume(const uint8_t * __restrict__ w, uint3
                 // of superblock 2 h + j / 2; the row's chunk starts sh bytes into its window
                 const uint32_t wrow = min(rbeg + 16 * t + r, rend - 1);
                 const uint32_t sh = ((uint32_t)(uintptr_t)w + wrow * RB + c * CB) & 15u;
-                const bool diag = (r >> 2) == j;
+                const bool diag = (r & 3) == j;
 #pragma unroll
                 for (uint32_t h = 0; h < 2; ++h) {
                     if (2 * h >= units) break;
@@ -342,33 +360,23 @@ __device__ __forceinline__ void cw_consume(const uint8_t * __restrict__ w, uint3
                         E[2 * l] = iq_apply(E[2 * l], n.x);
                         E[2 * l + 1] = iq_apply(E[2 * l + 1], n.y);
                     }
-                    const float db = iq_db(FMT, h2f(hd), w1);
+                    uint32_t db[4];
+                    cw_gather(__float_as_uint(iq_db(FMT, h2f(hd), w1)), db);
                     const v4i b0 = {(int)E[0], (int)E[1], (int)E[2], (int)E[3]}, b1 = {(int)E[4], (int)E[5], (int)E[6], (int)E[7]};
-                    const uint32_t b = 16 * h + 4 * j + k;
 #pragma unroll
-                    for (int gr = 0; gr < NG; ++gr) {
-                        // A as for Q8_0 below
-                        const lds32 ap = lp32(diag ? xs + (4 * gr + (r & 3)) * AROW + 36 * b + 4 : zr);
+                    for (int gr = 0; gr < NG; ++gr) {             // A as for Q8_0 below
+                        const lds32 ap = lp32(diag ? xs + (4 * gr + (r >> 2)) * AROW + 36 * (16 * h + 4 * j + k) + 4 : zr);
                         const v4i a0 = {(int)ap[0], (int)ap[1], (int)ap[2], (int)ap[3]};
                         const v4i a1 = {(int)ap[4], (int)ap[5], (int)ap[6], (int)ap[7]};
                         const u32x4a dx = *(const __attribute__((address_space(3))) u32x4a *)(uintptr_t)(
-                            xt + (b * NC + 4 * gr) * 4);
+                            xt + 32 * P::CU * (4 * gr + j) + 64 * h + 16 * k);
                         v4i d = __builtin_amdgcn_mfma_i32_16x16x64_i8(a0, b0, v4i{0, 0, 0, 0}, 0, 0, 0);
                         d = __builtin_amdgcn_mfma_i32_16x16x64_i8(a1, b1, d, 0, 0, 0);
-                        uint32_t m[4], f[4];
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) {
-                            m[i] = __float_as_uint(db * h2f(dx[i] & 0xFFFFu));
-                            f[i] = (uint32_t)d[i];
-                        }
-                        cw_transpose(m);                          // lane row j: column 4 gr + j, blocks t = 0..3
-                        cw_transpose(f);
-                        acc[gr] = fmaf(__uint_as_float(m[0]), (float)(int)f[0], acc[gr]);
-                        acc[gr] = fmaf(__uint_as_float(m[1]), (float)(int)f[1], acc[gr]);
-                        if (units > 2 * h + 1) {                  // (blocks 2 and 3 lie in the second superblock)
-                            acc[gr] = fmaf(__uint_as_float(m[2]), (float)(int)f[2], acc[gr]);
-                            acc[gr] = fmaf(__uint_as_float(m[3]), (float)(int)f[3], acc[gr]);
-                        }
+                        acc[gr] = fmaf(cw_fmul(db[0], dx[0], nz), (float)d[0], acc[gr]);
+                        acc[gr] = fmaf(cw_fmul(db[1], dx[1], nz), (float)d[1], acc[gr]);
+                        const float a2 = fmaf(cw_fmul(db[2], dx[2], nz), (float)d[2], acc[gr]);
+                        const float a3 = fmaf(cw_fmul(db[3], dx[3], nz), (float)d[3], a2);
+                        acc[gr] = units > 2 * h + 1 ? a3 : acc[gr];   // (blocks 2 and 3 lie in the second superblock)
                     }
                 }
             } else if constexpr (!KF) {
@@ -402,32 +410,27 @@ __device__ __forceinline__ void cw_consume(const uint8_t * __restrict__ w, uint3
                         }
                     }
                     const v4i b0 = {(int)B[0], (int)B[1], (int)B[2], (int)B[3]}, b1 = {(int)B[4], (int)B[5], (int)B[6], (int)B[7]};
-                    const bool diag = (r >> 2) == j;
+                    const bool diag = (r & 3) == j;
+                    uint32_t dw[4];
+                    cw_gather(W[O >> 2], dw);
+                    constexpr bool HI = (O & 2) != 0;
 #pragma unroll
                     for (int gr = 0; gr < NG; ++gr) {
-                        // A row n: column n % 4 of the group, non-zero on k-slice
-                        // n / 4 only, so lane row j receives its own block's dots
-                        const lds32 ap = lp32(diag ? xs + (4 * gr + (r & 3)) * AROW + 36 * (4 * j + K) + 4 : zr);
+                        // A row n: column n / 4 of the group, non-zero on k-slice
+                        // n % 4 only, so lane row j receives column j's dots with
+                        // the blocks t = 0..3 that lane rows 0..3 hold
+                        const lds32 ap = lp32(diag ? xs + (4 * gr + (r >> 2)) * AROW + 36 * (4 * j + K) + 4 : zr);
                         const v4i a0 = {(int)ap[0], (int)ap[1], (int)ap[2], (int)ap[3]};
                         const v4i a1 = {(int)ap[4], (int)ap[5], (int)ap[6], (int)ap[7]};
                         const u32x4a dx = *(const __attribute__((address_space(3))) u32x4a *)(uintptr_t)(
-                            xt + ((4 * j + K) * NC + 4 * gr) * 4);
+                            xt + 32 * P::CU * (4 * gr + j) + 16 * K);
                         v4i d = __builtin_amdgcn_mfma_i32_16x16x64_i8(a0, b0, v4i{0, 0, 0, 0}, 0, 0, 0);
                         d = __builtin_amdgcn_mfma_i32_16x16x64_i8(a1, b1, d, 0, 0, 0);
-                        uint32_t m[4], f[4];
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) {
-                            m[i] = __float_as_uint(cw_hmul<(O & 2) != 0>(W[O >> 2], dx[i], nz));
-                            f[i] = (uint32_t)d[i];
-                        }
-                        cw_transpose(m);                          // lane row j: column 4 gr + j, blocks t = 0..3
-                        cw_transpose(f);
-                        acc[gr] = fmaf(__uint_as_float(m[0]), (float)(int)f[0], acc[gr]);
-                        acc[gr] = fmaf(__uint_as_float(m[1]), (float)(int)f[1], acc[gr]);
-                        if (units > 1) {                          // (a half chunk: blocks 2 and 3 are not there)
-                            acc[gr] = fmaf(__uint_as_float(m[2]), (float)(int)f[2], acc[gr]);
-                            acc[gr] = fmaf(__uint_as_float(m[3]), (float)(int)f[3], acc[gr]);
-                        }
+                        acc[gr] = fmaf(cw_hmul<HI>(dw[0], dx[0], nz), (float)d[0], acc[gr]);
+                        acc[gr] = fmaf(cw_hmul<HI>(dw[1], dx[1], nz), (float)d[1], acc[gr]);
+                        const float a2 = fmaf(cw_hmul<HI>(dw[2], dx[2], nz), (float)d[2], acc[gr]);
+                        const float a3 = fmaf(cw_hmul<HI>(dw[3], dx[3], nz), (float)d[3], a2);
+                        acc[gr] = units > 1 ? a3 : acc[gr];       // (a half chunk: blocks 2 and 3 are not there)
                     }
                 };
                 switch (k) {
@@ -452,21 +455,22 @@ __device__ __forceinline__ void cw_consume(const uint8_t * __restrict__ w, uint3
                         hi[0][i] = (int)((qa[i] >> 4) & 0x0F0F0F0Fu);
                         hi[1][i] = (int)((qb[i] >> 4) & 0x0F0F0F0Fu);
                     }
-                    // 6-bit scales and mins of sub-blocks 2 j, 2 j + 1 (SWAR, fl_q4k_scale_min)
-                    const uint32_t wsc = j < 2 ? hd.y & 0x3F3F3F3Fu : (hd.w & 0x0F0F0F0Fu) | ((hd.y >> 2) & 0x30303030u);
+                    // the row's 6-bit scales, the mins of sub-blocks 2 j, 2 j + 1 (SWAR,
+                    // fl_q4k_scale_min)
+                    const uint32_t sc[2] = {hd.y & 0x3F3F3F3Fu, (hd.w & 0x0F0F0F0Fu) | ((hd.y >> 2) & 0x30303030u)};
                     const uint32_t wmn = j < 2 ? hd.z & 0x3F3F3F3Fu : ((hd.w >> 4) & 0x0F0F0F0Fu) | ((hd.z >> 2) & 0x30303030u);
-                    const uint32_t s16 = (wsc >> (16 * (j & 1))), m16 = (wmn >> (16 * (j & 1)));
-                    const int s0 = (int)(s16 & 0xFFu), s1 = (int)((s16 >> 8) & 0xFFu);
+                    const uint32_t m16 = (wmn >> (16 * (j & 1)));
                     const int n0 = (int)((m16 & 0xFFu) * 0x01010101u), n1 = (int)(((m16 >> 8) & 0xFFu) * 0x01010101u);
                     const v4i mv0 = {n0, n0, n0, n0}, mv1 = {n1, n1, n1, n1};
                     const float d = h2f(hd.x & 0xFFFFu), dmin = h2f(hd.x >> 16);
-                    const bool diag = (r >> 2) == j;
+                    const bool diag = (r & 3) == j;
 #pragma unroll
                     for (int gr = 0; gr < NG; ++gr) {
-                        // A row n: column n % 4 of the group, non-zero on k-slice n / 4
-                        // only, so lane row j receives its own sub-blocks' dots
+                        // A row n: column n / 4 of the group, non-zero on k-slice n % 4
+                        // only, so lane row j receives column j's dots with the
+                        // sub-blocks 2 i (d0) and 2 i + 1 (d1) of lane row i
                         const uint32_t xc = xs + 4 * gr * AROW + 292 * k;
-                        const lds32 ap = lp32(diag ? xc + (r & 3) * AROW + 36 + 64 * j : zr);
+                        const lds32 ap = lp32(diag ? xc + (r >> 2) * AROW + 36 + 64 * j : zr);
                         v4i a[4];
 #pragma unroll
                         for (int i = 0; i < 4; ++i) a[i] = v4i{(int)ap[4 * i], (int)ap[4 * i + 1], (int)ap[4 * i + 2], (int)ap[4 * i + 3]};
@@ -480,13 +484,13 @@ __device__ __forceinline__ void cw_consume(const uint8_t * __restrict__ w, uint3
                         dm = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[1], mv0, dm, 0, 0, 0);
                         dm = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[2], mv1, dm, 0, 0, 0);
                         dm = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[3], mv1, dm, 0, 0, 0);
-                        int pr[4], pm[4];
+                        int ti = 0;
 #pragma unroll
                         for (int i = 0; i < 4; ++i) {
-                            pr[i] = __mul24(s0, d0[i]) + __mul24(s1, d1[i]);
-                            pm[i] = dm[i];
+                            const uint32_t s2 = sc[i >> 1] >> (16 * (i & 1));
+                            ti += __mul24((int)(s2 & 0xFFu), d0[i]) + __mul24((int)((s2 >> 8) & 0xFFu), d1[i]);
                         }
-                        const int ti = cw_rowsum(pr), tm = cw_rowsum(pm);   // lane row j: column 4 gr + j
+                        const int tm = (dm[0] + dm[1]) + (dm[2] + dm[3]);
                         const float dk = __uint_as_float(*lp32(xc + j * AROW));
                         acc[gr] = fmaf(d * dk, (float)ti, acc[gr]);
                         acc[gr] = fmaf(-(dmin * dk), (float)tm, acc[gr]);
@@ -511,44 +515,42 @@ __device__ __forceinline__ void cw_consume(const uint8_t * __restrict__ w, uint3
                     const uint32_t SC[4] = {alignb(sp[1], sp[0], s2), alignb(sp[2], sp[1], s2), alignb(sp[3], sp[2], s2),
                                             alignb(sp[4], sp[3], s2)};
                     const float d = h2f((s2 ? sp[4] >> 16 : sp[4]) & 0xFFFFu);
+                    // 4 (q - 32) per byte: the six bits at the top, the highest one
+                    // inverted (qh: once for its four groups)
                     uint32_t Bv[8][2];
 #pragma unroll
                     for (int m = 0; m < 8; ++m) {                 // half m / 4, group m % 4
                         const int hh = m >> 2, gg = m & 3;
 #pragma unroll
                         for (int u = 0; u < 2; ++u) {
-                            const uint32_t ql = W[2 * hh + (gg & 1)][u], qh = W[4 + hh][u];
-                            const uint32_t nib = gg < 2 ? ql & 0x0F0F0F0Fu : (ql >> 4) & 0x0F0F0F0Fu;
-                            const uint32_t hb = ((qh >> (2 * gg)) & 0x03030303u) << 4;
-                            Bv[m][u] = ((nib | hb) + 0x60606060u) ^ 0x80808080u;   // q - 32 per byte
+                            const uint32_t ql = W[2 * hh + (gg & 1)][u], qh = W[4 + hh][u] ^ 0xAAAAAAAAu;
+                            const uint32_t nib = (gg < 2 ? ql << 2 : ql >> 2) & 0x3C3C3C3Cu;
+                            Bv[m][u] = nib | ((qh << (6 - 2 * gg)) & 0xC0C0C0C0u);
                         }
                     }
 #pragma unroll
                     for (int gr = 0; gr < NG; ++gr) {
-                        // A row n: column 8 gr + n % 8, non-zero on the k-slices of
-                        // sub-block 2 m + n / 8 only, so lane rows 0-1 (2-3) receive
-                        // that sub-block's dots
-                        const uint32_t xc = xs + ((8 * gr + (r & 7)) & (NC - 1)) * AROW + 292 * k + 8 * j;
-                        const lds32 ap = lp32((r >> 3) == (j >> 1) ? xc + 36 : zr);
-                        int ia[4] = {0, 0, 0, 0};
+                        // A row n: column 8 gr + n / 2, non-zero on the k-slices of
+                        // sub-block 2 m + n % 2 only, so lane row j receives the dots of
+                        // columns 2 j (dd[0], dd[1]) and 2 j + 1 with both sub-blocks
+                        const uint32_t xc = xs + ((8 * gr + (r >> 1)) & (NC - 1)) * AROW + 292 * k + 8 * j;
+                        const lds32 ap = lp32((r & 1) == (j >> 1) ? xc + 36 : zr);
+                        int ia[2] = {0, 0};
 #pragma unroll
                         for (int m = 0; m < 8; ++m) {
                             const v4i dd = __builtin_amdgcn_mfma_i32_16x16x32_i8(
                                 (long)(((uint64_t)ap[8 * m + 1] << 32) | ap[8 * m]),
                                 (long)(((uint64_t)Bv[m][1] << 32) | Bv[m][0]), v4i{0, 0, 0, 0}, 0, 0, 0);
-                            // scale of sub-block 2 m + j / 2
-                            const int sc = (int)(int8_t)(SC[m >> 1] >> (16 * (m & 1) + 8 * (j >> 1)));
-#pragma unroll
-                            for (int i = 0; i < 4; ++i) ia[i] += __mul24(sc, dd[i]);
+                            const int s0 = (int)(int8_t)(SC[m >> 1] >> (16 * (m & 1)));
+                            const int s1 = (int)(int8_t)(SC[m >> 1] >> (16 * (m & 1) + 8));
+                            ia[0] += __mul24(s0, dd[0]) + __mul24(s1, dd[1]);
+                            ia[1] += __mul24(s0, dd[2]) + __mul24(s1, dd[3]);
                         }
-                        // the two sub-blocks' sums: columns 4 (j & 1) + 2 (j >> 1) + {0, 1}
-                        const auto u = __builtin_amdgcn_permlane32_swap((uint32_t)ia[0], (uint32_t)ia[2], false, false);
-                        const auto v = __builtin_amdgcn_permlane32_swap((uint32_t)ia[1], (uint32_t)ia[3], false, false);
-                        const uint32_t c0 = (8 * gr + 4 * (j & 1) + 2 * (j >> 1)) & (NC - 1);
+                        const uint32_t c0 = (8 * gr + 2 * j) & (NC - 1);
                         const float dk0 = __uint_as_float(*lp32(xs + c0 * AROW + 292 * k));
                         const float dk1 = __uint_as_float(*lp32(xs + (c0 + 1) * AROW + 292 * k));
-                        acc[2 * gr] = fmaf(d * dk0, (float)(int)(u[0] + u[1]), acc[2 * gr]);
-                        acc[2 * gr + 1] = fmaf(d * dk1, (float)(int)(v[0] + v[1]), acc[2 * gr + 1]);
+                        acc[2 * gr] = fmaf(d * dk0, (float)(ia[0] >> 2), acc[2 * gr]);
+                        acc[2 * gr + 1] = fmaf(d * dk1, (float)(ia[1] >> 2), acc[2 * gr + 1]);
                     }
                 }
             }
@@ -585,7 +587,7 @@ __device__ __forceinline__ void cw_rows(uint32_t rows, uint32_t g, uint32_t G, u
 }
 
 template <int FMT, int NC, int D>
-__global__ __launch_bounds__(64 * CW_WAVES) void k_dot_cw(DotArgs a) {
+__global__ __launch_bounds__(64 * CW_WAVES, 4) void k_dot_cw(DotArgs a) {
     extern __shared__ __attribute__((aligned(16))) uint8_t cw_sm[];
     const uint8_t * w = a.w + (a.id_slot ? (size_t)(*a.id_slot) * a.estride : 0);
     const CwColsStrided C{a.x, a.y, a.xstride, a.ystride};
@@ -597,7 +599,7 @@ __global__ __launch_bounds__(64 * CW_WAVES) void k_dot_cw(DotArgs a) {
 // Grouped experts: the routed experts share the grid (moe_assign); the
 // workgroup streams its rows of its expert once per NC of the expert's pairs.
 template <int FMT, int NC, int D>
-__global__ __launch_bounds__(64 * CW_WAVES) void k_moe_cw(MoeArgs a) {
+__global__ __launch_bounds__(64 * CW_WAVES, 4) void k_moe_cw(MoeArgs a) {
     extern __shared__ __attribute__((aligned(16))) uint8_t cw_sm[];
     __shared__ uint32_t pairs[256], rids[256], npairs, cxi[NC], cyi[NC];
     const uint32_t tid = threadIdx.x;
