@@ -596,12 +596,35 @@ __global__ __launch_bounds__(64 * CW_WAVES, 4) void k_dot_cw(DotArgs a) {
     cw_body<FMT, NC, D>(w, a.cols, C, a.nx, rbeg, rend, cw_sm);
 }
 
+// Ring depth within `lds` bytes and the vmcnt range.  Up to one 16-row tile per
+// CU: a workgroup alone on its CU, the ring deep (Q8_0 4096x14336 with 4 columns
+// 14.9 us, 17.7 with 3 stages; Q6_K with 8 columns 15.9 / 18.4).  More tiles: 3
+// stages and two workgroups per CU, or three where 4 columns' stages are small
+// (Q4_K 28672x4096 with 3 columns 15.3 us, 16.6 with two workgroups and a deep
+// ring; Q8_0 11264x2048 7.6 / 8.8; Q6_K's stages are larger: 25.0 with two,
+// 28.9 with three).
+template <int FMT, int NC> constexpr int cw_depth(int most, size_t lds) {
+    int d = 2;
+    while (d < most && cw_smem<FMT, NC>(d + 1) <= lds && (d - 1) * (int)CwPlan<FMT, NC>::NT <= 60) ++d;
+    return d;
+}
+constexpr size_t CW_LDS1 = 150 * 1024, CW_LDS2 = 80 * 1024;       // one or two workgroups per CU
 // Grouped experts: the routed experts share the grid (moe_assign); the
-// workgroup streams its rows of its expert once per NC of the expert's pairs.
-template <int FMT, int NC, int D>
+// workgroup streams its rows of its expert once for up to 16 of the expert's
+// pairs, in the smallest of the 4-, 8- and 16-column forms that holds them: the
+// counts differ from expert to expert (8 tokens, 2 of 8 experts: 2 on average,
+// often 5), and one form for all of them, sized for the average, read the
+// weights of every fuller expert twice.
+template <int FMT, int NC> constexpr int cw_moe_depth() { return cw_depth<FMT, NC>(3, CW_LDS2); }
+template <int FMT> constexpr size_t cw_moe_smem() {
+    size_t m = cw_smem<FMT, 4>(cw_moe_depth<FMT, 4>());
+    for (size_t n : {cw_smem<FMT, 8>(cw_moe_depth<FMT, 8>()), cw_smem<FMT, 16>(cw_moe_depth<FMT, 16>())}) m = n > m ? n : m;
+    return m;
+}
+template <int FMT>
 __global__ __launch_bounds__(64 * CW_WAVES, 4) void k_moe_cw(MoeArgs a) {
     extern __shared__ __attribute__((aligned(16))) uint8_t cw_sm[];
-    __shared__ uint32_t pairs[256], rids[256], npairs, cxi[NC], cyi[NC];
+    __shared__ uint32_t pairs[256], rids[256], npairs, cxi[16], cyi[16];
     const uint32_t tid = threadIdx.x;
     if (tid == 0) npairs = 0;
     const uint32_t * ids = moe_route(a, rids);
@@ -614,16 +637,19 @@ __global__ __launch_bounds__(64 * CW_WAVES, 4) void k_moe_cw(MoeArgs a) {
     const uint8_t * w = a.w + (size_t)e * a.estride;
     uint32_t rbeg, rend;
     cw_rows(a.rows, g, G, rbeg, rend);
-    for (uint32_t p0 = 0; p0 < np; p0 += NC) {
-        const uint32_t nx = min((uint32_t)NC, np - p0);
-        if (tid < NC) {
+    if (rbeg >= rend) return;
+    for (uint32_t p0 = 0; p0 < np; p0 += 16) {
+        const uint32_t nx = min(16u, np - p0);
+        if (tid < 16) {
             const uint32_t ts = pairs[p0 + (tid < nx ? tid : 0)];
             cxi[tid] = a.x_per_slot ? ts : ts / a.top_k;
             cyi[tid] = ts;
         }
         __syncthreads();
         const CwColsMoe C{a.x, a.y, a.xstride, a.ystride, cxi, cyi};
-        if (rbeg < rend) cw_body<FMT, NC, D>(w, a.cols, C, nx, rbeg, rend, cw_sm);
+        if (nx <= 4) cw_body<FMT, 4, cw_moe_depth<FMT, 4>()>(w, a.cols, C, nx, rbeg, rend, cw_sm);
+        else if (nx <= 8) cw_body<FMT, 8, cw_moe_depth<FMT, 8>()>(w, a.cols, C, nx, rbeg, rend, cw_sm);
+        else cw_body<FMT, 16, cw_moe_depth<FMT, 16>()>(w, a.cols, C, nx, rbeg, rend, cw_sm);
         __syncthreads();
     }
 }
@@ -640,19 +666,6 @@ static bool cw_takes(int fmt, const void * w, uint64_t estride, const void * x, 
     return !((uintptr_t)w & al) && !(estride & al);
 }
 
-// Ring depth within `lds` bytes and the vmcnt range.  Up to one 16-row tile per
-// CU: a workgroup alone on its CU, the ring deep (Q8_0 4096x14336 with 4 columns
-// 14.9 us, 17.7 with 3 stages; Q6_K with 8 columns 15.9 / 18.4).  More tiles: 3
-// stages and two workgroups per CU, or three where 4 columns' stages are small
-// (Q4_K 28672x4096 with 3 columns 15.3 us, 16.6 with two workgroups and a deep
-// ring; Q8_0 11264x2048 7.6 / 8.8; Q6_K's stages are larger: 25.0 with two,
-// 28.9 with three).
-template <int FMT, int NC> constexpr int cw_depth(int most, size_t lds) {
-    int d = 2;
-    while (d < most && cw_smem<FMT, NC>(d + 1) <= lds && (d - 1) * (int)CwPlan<FMT, NC>::NT <= 60) ++d;
-    return d;
-}
-constexpr size_t CW_LDS1 = 150 * 1024, CW_LDS2 = 80 * 1024;       // one or two workgroups per CU
 template <int FMT, int NC, int D>
 static int cw_go(const DotArgs & a, uint32_t G, hipStream_t s) {
     constexpr size_t smb = cw_smem<FMT, NC>(D);
@@ -734,23 +747,15 @@ int launch_dot_cw(int fmt, const DotArgs & a, hipStream_t s) {
     }
 }
 
-template <int FMT, int NC>
-static int cw_moe_go(const MoeArgs & a, hipStream_t s) {
-    constexpr int D = cw_depth<FMT, NC>(3, CW_LDS2);
-    constexpr size_t smb = cw_smem<FMT, NC>(D);
+template <int FMT> static int cw_moe(const MoeArgs & a, hipStream_t s) {
+    constexpr size_t smb = cw_moe_smem<FMT>();
     const uint32_t wgs = (tune().cw_wpc ? tune().cw_wpc : 2) * (uint32_t)num_cus();
-    const void * kern = (const void *)k_moe_cw<FMT, NC, D>;
+    const void * kern = (const void *)k_moe_cw<FMT>;
     if (int rc = lds_fits(kern, smb, "k_moe_cw")) return rc;
     (void)hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smb);
-    hipLaunchKernelGGL((k_moe_cw<FMT, NC, D>), dim3(wgs), dim3(64 * CW_WAVES), smb, s, a);
+    hipLaunchKernelGGL((k_moe_cw<FMT>), dim3(wgs), dim3(64 * CW_WAVES), smb, s, a);
     return hip_check(hipGetLastError(), "k_moe_cw launch");
 }
-template <int FMT> static int cw_moe(const MoeArgs & a, hipStream_t s) {
-    const uint32_t pairs = a.ntok * a.top_k, per = (pairs + moe_rows(a) - 1) / moe_rows(a);
-    return per <= 4 ? cw_moe_go<FMT, 4>(a, s) : per <= 8 ? cw_moe_go<FMT, 8>(a, s) : cw_moe_go<FMT, 16>(a, s);
-}
-// Columns per pass: what an active expert has on average (an expert with more
-// takes further passes over its weights).
 int launch_moe_cw(int fmt, const MoeArgs & a, hipStream_t s) {
     if (!cw_on(fmt)) return FLH_ERR_UNSUPPORTED;
     const uint64_t pairs = (uint64_t)a.ntok * a.top_k;
