@@ -688,12 +688,12 @@ template <int FMT> static int cw_launch(const DotArgs & a, hipStream_t s) {
 // Whether a matrix with nx columns is faster here than on the format's other
 // kernel (us here / there):
 //  * Q4_K against k_dot_mfma, whose tiles are 16 x 144-byte pieces but which
-//    stages the columns once per workgroup: 4 columns 14336x4096 9.7 / 10.6,
-//    6144x4096 6.3 / 7.2, 4096x14336 10.0 / 11.7; 8 columns 4096x14336 12.4 /
-//    14.6, 14336x4096 11.6 / 11.8, 28672x4096 19.2 / 17.7; 16 columns 4096^2
-//    7.7 / 8.1, 6144x4096 12.3 / 9.6, 28672x4096 32 / 21.6 (the columns are as
-//    many bytes as the weights there), and where that kernel needs several
-//    passes 27648x5120 38 / 46, 8192x8192 20 / 25.
+//    stages the columns once per workgroup: 4 columns 14336x4096 9.6 / 10.6,
+//    4096x14336 9.2 / 11.7; 8 columns 6144x4096 6.6 / 7.9, 4096x14336 11.5 / 14.6,
+//    14336x4096 10.8 / 11.6, 28672x4096 17.1 / 17.9; 16 columns 4352x1792 6.2 /
+//    6.8, 6144x4096 8.4 / 9.6, 9216x3840 13.2 / 13.0, 14336x4096 14.3 / 14.5, but
+//    28672x4096 23.1 / 21.7 (the columns are as many bytes as the weights), and
+//    where that kernel needs several passes 27648x5120 38 / 46, 8192x8192 20 / 25.
 //  * Q6_K against the streaming kernel: 2 columns 14336x4096 14.5 / 12.1,
 //    4096^2 7.4 / 6.5, 4096x14336 15.7 / 16.5; 3 columns 14336x4096 14.5 / 16.2,
 //    6144x4096 9.2 / 9.1; 8 columns 14336x4096 15.7 / 21.7, 4096x14336 15.9 / 40;
@@ -717,7 +717,7 @@ template <int FMT> static int cw_launch(const DotArgs & a, hipStream_t s) {
 //    6.5 / 8.7, 10.2 / 44; one column of few rows, 1024x2816: 5.4 / 5.1.
 static bool cw_wins(int fmt, uint32_t rows, uint32_t cols, uint32_t nx) {
     const uint32_t T = (rows + 15) / 16, cus = (uint32_t)num_cus();
-    if (fmt == FMT_Q4_K) return nx <= 4 || (nx <= 8 ? rows <= 16384 : T <= cus || cols > 4096);
+    if (fmt == FMT_Q4_K) return nx <= 8 || rows <= 16384 || cols > 4096;
     if (fmt == FMT_Q6_K) return nx > 2 || cols > 8192;
     if (cw_iq(fmt)) {
         if (nx == 1) return cols > 16128 || ((cols & 2047) && rows >= 2048);
