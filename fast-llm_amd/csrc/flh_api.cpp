@@ -516,6 +516,10 @@ int flh_graph_launch(void * ge, void * stream) {
     const graph_handle * h = (const graph_handle *)ge;
     if (!h) return set_error(FLH_ERR_ARG, "null graph");
     if (h->exec) return hip_check(hipGraphLaunch(h->exec, (hipStream_t)stream), "hipGraphLaunch");
+    // one replay at a time: threads that replay onto one stream get whole graphs
+    // in some order, as from the runtime's launch, not their kernels interleaved
+    static std::mutex whole;
+    std::lock_guard<std::mutex> lock(whole);
     for (const hipKernelNodeParams & k : h->chain)
         if (int rc = hip_check(hipLaunchKernel(k.func, k.gridDim, k.blockDim, k.kernelParams, k.sharedMemBytes,
                                                (hipStream_t)stream), "graph kernel launch")) return rc;
