@@ -177,7 +177,9 @@ int flh_event_destroy(void * event);
 /* HIP graph capture of work issued on one stream (replaces the reference's
  * persistent-kernel launch amortisation, src/runtime/gpu_exec.cu:156-344,
  * for a frozen graph: capture once, replay per token).  Every kernel of
- * this library is capture-safe (no hipMemsetAsync, no host syncs). */
+ * this library is capture-safe (no hipMemsetAsync, no host syncs).  The
+ * handle is this library's own (a short chain of kernels is replayed kernel by
+ * kernel, anything else as the runtime's graph): launch and destroy it here. */
 int flh_graph_capture_begin(void * stream);
 int flh_graph_capture_end(void * stream, void ** graph_exec);
 int flh_graph_launch(void * graph_exec, void * stream);
