@@ -136,8 +136,8 @@ void load_tune() {
     if (const char * e = getenv("FLH_NO_Q6MF")) t.no_q6mf = atoi(e) != 0;
     if (const char * e = getenv("FLH_SBL_NX_DEP")) t.sbl_nx_dep = (uint32_t)atoi(e);
     if (const char * e = getenv("FLH_CW")) {
-        unsigned m = 0, w = 0;
-        if (sscanf(e, "%u,%u", &m, &w) >= 1) { t.cw = m; t.cw_wpc = w; }
+        unsigned m = 0, w = 0, g = 0;
+        if (sscanf(e, "%u,%u,%u", &m, &w, &g) >= 1) { t.cw = m; t.cw_wpc = w; t.cw_gmax = g; }
     }
     for (const char * v : {"FLH_MFMA_PRO", "FLH_MFMA_TUNE", "FLH_MFMA_XC", "FLH_MFMA_OWN", "FLH_MFMA_MIN_COLS"})
         t.mf_forced = t.mf_forced || getenv(v);

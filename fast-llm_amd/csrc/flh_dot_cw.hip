@@ -749,7 +749,10 @@ int launch_dot_cw(int fmt, const DotArgs & a, hipStream_t s) {
 
 template <int FMT> static int cw_moe(const MoeArgs & a, hipStream_t s) {
     constexpr size_t smb = cw_moe_smem<FMT>();
-    const uint32_t wgs = (tune().cw_wpc ? tune().cw_wpc : 2) * (uint32_t)num_cus();
+    uint32_t wgs = (tune().cw_wpc ? tune().cw_wpc : 2) * (uint32_t)num_cus();
+    if (tune().cw_gmax && wgs > tune().cw_gmax) wgs = tune().cw_gmax;
+    // a workgroup per expert at least (moe_assign); a partitioned device has as few as 32 CUs
+    if (wgs < moe_rows(a)) wgs = moe_rows(a);
     const void * kern = (const void *)k_moe_cw<FMT>;
     if (int rc = lds_fits(kern, smb, "k_moe_cw")) return rc;
     (void)hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smb);

@@ -98,9 +98,10 @@ struct Tune {
     uint32_t sbl = 1, sbl_w = 0, sbl_wpc = 0, sbl_gmax = 0, sbl_pre = 0;
     uint32_t sbl_nx_dep = 0;            // FLH_SBL_NX_DEP: ring stages of the several-column kernel (0: planned)
     bool mf_forced = false;             // any FLH_MFMA_* override: Q4_K stays on that kernel
-    // chain-per-wave matrix-core kernel, FLH_CW = "mode[,wgs_per_cu]": 0 never,
-    // 1 where it is the faster one, 2 wherever it takes the shape; wgs_per_cu 0: planned
-    uint32_t cw = 1, cw_wpc = 0;
+    // chain-per-wave matrix-core kernel, FLH_CW = "mode[,wgs_per_cu[,max_wgs]]": 0 never,
+    // 1 where it is the faster one, 2 wherever it takes the shape; wgs_per_cu 0: planned;
+    // max_wgs: the grouped launch's grid as on a device of fewer CUs (0: all)
+    uint32_t cw = 1, cw_wpc = 0, cw_gmax = 0;
     uint32_t gguf_threads = 0;          // FLH_GGUF_THREADS: host copy threads of an upload (0: all, <= 16)
 };
 const Tune & tune();

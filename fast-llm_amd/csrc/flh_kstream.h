@@ -834,7 +834,9 @@ __device__ __forceinline__ const uint32_t * moe_route(const MoeArgs & a, uint32_
 // expert j (the j-th smallest id) taking workgroups [ceil(jB/n),
 // ceil((j+1)B/n)); returns e = n_expert when nothing is routed, else e and
 // this workgroup's index g among its expert's G.  Every workgroup computes the
-// same split from the same ids, so none idles on an unrouted expert.
+// same split from the same ids, so none idles on an unrouted expert.  B must be
+// at least n, or the experts between two workgroups' are left out: a launch has
+// moe_rows() workgroups or more.
 // Contains barriers.
 __device__ __forceinline__ uint32_t moe_assign(const uint32_t * ids, uint32_t nids, uint32_t n_expert, uint32_t b,
                                                uint32_t B, uint32_t & g, uint32_t & G) {
