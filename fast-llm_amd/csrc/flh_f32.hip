@@ -754,7 +754,9 @@ static int launch_f32(bool fast, int fmt, const DotArgs & a, hipStream_t s) {
                          fmt == FMT_IQ3_XXS;
     // F32, one column or a small matrix: one workgroup per row and group of 4
     // columns, all columns in one launch
-    if (fast && fmt == FMT_F32 && a.nx <= 16 && a.rows <= 0x7FFFFFFFu &&
+    // (a launch holds fewer than 2^32 threads: 2^24 rows and more stay with
+    // k_dot_f32row, 16 rows a workgroup)
+    if (fast && fmt == FMT_F32 && a.nx <= 16 && a.rows < (1u << 24) &&
         (a.nx == 1 || (uint64_t)a.rows * ((a.nx + 3) / 4) <= F32S_MAX_WG)) {
         const uint32_t nxt = a.nx == 1 ? 1 : a.nx == 2 ? 2 : 4;
         const size_t smem = (size_t)nxt * 16 * F32S_MP * 4;

@@ -29,3 +29,24 @@ def test_f32_small_bitwise(flh, orc, gpu, rows, cols, nx):
     want = y0.copy()
     orc.stream_dot(F32, w, rows, cols, hx, want, nx=nx, xstride=st, ystride=rows, fast=True, threads=8)
     assert np.array_equal(bits(dy.download(np.float32, y0.size, gpu)), bits(want))
+
+
+@pytest.mark.parametrize("rows", [(1 << 24) - 1, 1 << 24, (1 << 24) + 37])
+def test_f32_rows_past_one_launch(flh, orc, gpu, rows):
+    """2^24 rows of one column: a workgroup of 256 threads per row is more than a
+    launch holds.  The matrix repeats 4099 rows, and so do its outputs."""
+    say("f32 rows", rows)
+    cols, rep = 16, 4099
+    rng = np.random.default_rng(rows)
+    w = normal_weights(rep, cols, rng, std=0.5)
+    xs = activations(1, cols, rng)
+    dx, hx = dev_cols(flh, gpu, xs, col_stride_floats(cols))
+    dw = flh.DeviceBuffer.from_array(np.resize(w, (rows, cols)), gpu)
+    dy = flh.DeviceBuffer(4 * rows)
+    dy.zero(gpu)
+    flh.stream_dot(F32, dw, rows, cols, dx, dy, gpu)
+    want = np.zeros(rep, np.float32)
+    orc.stream_dot(F32, w.view(np.uint8).reshape(-1), rep, cols, hx, want, fast=True, threads=8)
+    got = dy.download(np.float32, rows, gpu)
+    dw.close()
+    assert np.array_equal(bits(got), bits(np.resize(want, rows)))
