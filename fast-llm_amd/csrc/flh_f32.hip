@@ -10,7 +10,7 @@
 //    dot_row_fast / dot_row_fast_q8_0 / dot_row_fast_dequant, bitwise: the
 //    256-element chunk formats (Q4_K, Q6_K -- the reference GPU masks' Q6_K
 //    route --, Q5_0, IQ2_XXS, IQ3_XXS) on one wave per row (k_dot_fastk),
-//    Q8_0 and several columns of a large F32 matrix on 16 lanes per row
+//    Q8_0 and F32 matrices of many short rows or with several columns on 16 lanes per row
 //    (k_dot_f32row), other F32 (e.g. an MoE router) on a workgroup per row
 //    (k_dot_f32small).
 //  * ROUTER_SEL / SILU_MUL / WMERGE / MERGE: the reference's single-thread
@@ -633,7 +633,7 @@ __global__ __launch_bounds__(256) void k_dot_f32row(DotArgs a, uint32_t T) {
     }
 }
 
-// F32 rows, one column, or a small matrix (an MoE router) and any: one
+// F32 rows, few (an MoE router) or long (f32_small below): one
 // workgroup per (row, group of up to 4 columns).  k_dot_f32row gives a small
 // matrix 16 rows per workgroup -- a handful of workgroups, each waiting for a
 // chain of load round trips (8 x 4096: 10.3 us, 26 us with 4 columns).  Here
@@ -736,14 +736,23 @@ __global__ void k_dot_canon(int fmt, DotArgs a) {
     *y = *y + v;
 }
 
-// Workgroups (rows x groups of 4 columns) up to which several columns of an
-// F32 matrix take k_dot_f32small, every column group reading the row anew.
-// k_dot_f32row / k_dot_f32small, us: 64 x 2048 with 4 columns 13.9 / 3.4, with
-// 16 55 / 3.5, 8 x 4096 with 8 49 / 4.5, 1024 x 4096 with 4 26 / 11.5, 2048 x
-// 1024 with 4 9.8 / 8.3; 4096 x 4096 with 4 29 / 35, 16384 x 1024 with 4 21 / 55.
-// One column takes it at any size: 8 x 4096 10.3 / 3.5, 4096 x 4096 18.8 /
-// 14.3, 16384 x 4096 58 / 46, 16384 x 1024 18.2 / 17.7.
-constexpr uint64_t F32S_MAX_WG = 2048;
+// Whether an F32 matrix takes k_dot_f32small (a workgroup per row and group of up
+// to 4 columns, each reading the row anew) and not k_dot_f32row (16 rows a
+// workgroup; us there / here).  A workgroup costs about 0.65 ns of the chip
+// however short its row: it wins where the rows are few (the chip is filled sooner)
+// or long.  One column: 8x4096 10.2 / 3.9, 2048x64 4.0 / 3.7, 4096x64 4.1 / 4.9,
+// 65536x256 20 / 47; 4096x768 5.5 / 5.5, 8192x768 7.7 / 9.4, 16384x1024 18.5 / 17.5,
+// 32768x1024 30.9 / 31.7, 65536x1536 69 / 73; 65536x2048 93 / 85, 262144x2048 337 /
+// 330, 262144x4096 764 / 677.  Several: 64x2048 with 4 columns 14.3 / 3.6, with 16 56
+// / 3.8, 2048x1024 with 3 / 4 9.0 / 7.8, 10.2 / 8.1, 2048x512 with 2 / 3 5.5 / 4.7, 6.7 /
+// 6.7, 2048x64 with 2 / 3 / 4 4.9 / 4.6, 5.1 / 6.5, 5.9 / 6.7, 1280x64 with 3 5.1 / 5.1;
+// past 2048 workgroups 4096x4096 with 4 29 / 35, 16384x1024 with 4 21 / 55.  (A launch
+// holds fewer than 2^32 threads: 2^24 rows are k_dot_f32row's.)
+static bool f32_small(uint32_t rows, uint32_t cols, uint32_t nx) {
+    if (rows >= (1u << 24)) return false;
+    if (nx == 1) return rows <= 2048 || cols >= 2048 || (cols >= 1024 ? rows <= 16384 : cols >= 768 && rows <= 4096);
+    return (uint64_t)rows * ((nx + 3) / 4) <= (cols < 512 && (nx == 3 || nx == 4) ? 1280u : 2048u);
+}
 
 static int launch_f32(bool fast, int fmt, const DotArgs & a, hipStream_t s) {
     if (fmt < FMT_F32 || fmt > FMT_IQ3_XXS)
@@ -752,12 +761,9 @@ static int launch_f32(bool fast, int fmt, const DotArgs & a, hipStream_t s) {
     if (n == 0) return FLH_OK;
     const bool chunked = fmt == FMT_Q4_K || fmt == FMT_Q6_K || fmt == FMT_Q5_0 || fmt == FMT_IQ2_XXS ||
                          fmt == FMT_IQ3_XXS;
-    // F32, one column or a small matrix: one workgroup per row and group of 4
-    // columns, all columns in one launch
-    // (a launch holds fewer than 2^32 threads: 2^24 rows and more stay with
-    // k_dot_f32row, 16 rows a workgroup)
-    if (fast && fmt == FMT_F32 && a.nx <= 16 && a.rows < (1u << 24) &&
-        (a.nx == 1 || (uint64_t)a.rows * ((a.nx + 3) / 4) <= F32S_MAX_WG)) {
+    // F32, few or long rows: one workgroup per row and group of 4 columns, all
+    // columns in one launch
+    if (fast && fmt == FMT_F32 && a.nx <= 16 && f32_small(a.rows, a.cols, a.nx)) {
         const uint32_t nxt = a.nx == 1 ? 1 : a.nx == 2 ? 2 : 4;
         const size_t smem = (size_t)nxt * 16 * F32S_MP * 4;
         const void * kern = nxt == 1 ? (const void *)k_dot_f32small<1> : nxt == 2 ? (const void *)k_dot_f32small<2>
@@ -812,7 +818,7 @@ static int launch_f32(bool fast, int fmt, const DotArgs & a, hipStream_t s) {
         const dim3 gw((a.rows + 15) / 16);
         const uint32_t slots = a.nx == 1 ? 0 : a.nx == 2 ? 1 : 2;
         static const void * const kf32[3] = {
-            (const void *)k_dot_f32row<FMT_F32, 2, 4>, (const void *)k_dot_f32row<FMT_F32, 2, 4>,
+            (const void *)k_dot_f32row<FMT_F32, 1, 4>, (const void *)k_dot_f32row<FMT_F32, 2, 4>,
             (const void *)k_dot_f32row<FMT_F32, 4, 2>};
         static const void * const kq8[3] = {
             (const void *)k_dot_f32row<FMT_Q8_0, 1, 4>, (const void *)k_dot_f32row<FMT_Q8_0, 2, 4>,
