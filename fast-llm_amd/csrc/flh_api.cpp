@@ -9,7 +9,9 @@
 #include <string>
 #include <vector>
 #include <atomic>
+#include <memory>
 #include <mutex>
+#include <unordered_map>
 #include "../../include/fastllm_hip.h"
 #include "flh_common.h"
 #include "flh_internal.h"
@@ -296,27 +298,64 @@ static void merge_tiles(const flh_task * t, uint32_t n, uint32_t & i, DotArgs & 
 
 using namespace flh;
 
+// The streams made by flh_stream_create.  (Never destroyed: threads may outlive
+// the statics.)
+namespace flh {
+namespace {
+struct StreamTurns {
+    std::shared_mutex m;
+    std::unordered_map<void *, std::shared_ptr<StreamTurn::State>> by_stream;
+};
+StreamTurns & turns() {
+    static StreamTurns * t = new StreamTurns();
+    return *t;
+}
+}  // namespace
+
+StreamTurn::StreamTurn(void * stream, bool whole) : whole_(whole) {
+    {
+        StreamTurns & t = turns();
+        std::shared_lock<std::shared_mutex> l(t.m);
+        const auto it = t.by_stream.find(stream);
+        if (it != t.by_stream.end()) st_ = it->second;
+    }
+    if (!st_) return;
+    std::lock_guard<std::mutex> l(st_->gate);                     // a waiting replay is next: calls that go on overlapping cannot keep it out
+    if (whole_) st_->m.lock();
+    else st_->m.lock_shared();
+}
+StreamTurn::~StreamTurn() {
+    if (!st_) return;
+    if (whole_) st_->m.unlock();
+    else st_->m.unlock_shared();
+}
+}  // namespace flh
+
 struct flh_arena {
     uint8_t * base;
     size_t cap, used;
 };
 
-// A captured graph: the runtime's executable form, or, for a short chain of
-// kernels (a few layers' launches), the kernels themselves, launched one by
-// one.  The runtime's graph launch adds about 6 us on the device to every
-// replay (n kernels of 1.5 us: 7.7 + 1.53 n us) and 13 us or more on the host;
-// one by one they cost 2.26 us of host time each.  So the line: 1 / 4 / 8 / 12 /
-// 16 kernels of 2.6 us 2.9 / 10.8 / 21.7 / 32.6 / 43.4 us here, 15.8 / 17.5 /
-// 27.9 / 38.3 / 48.7 us as a graph; of 1.5 us 3.2 / 9.8 / 18.2 / 27.4 / 36.8 against
-// 16.6 / 13.9 / 20.0 / 26.1 / 32.2 (this library's shortest kernels take 1.8-2.2
-// us).  Longer chains and anything but a chain of kernels keep the runtime's form.
+// A captured graph: the runtime's executable form and, for a chain of at most
+// five kernels, the kernels themselves, which are launched one by one on a
+// stream of this library's own (see flh_graph_launch).  The runtime's graph
+// launch adds about 6 us on the device to every replay and 16-18 us on the
+// host; a launch costs 2.6 us of host time, more where many are queued or
+// follow a wait.  us a replay in a row / us a replay that is waited for, one by
+// one against the runtime's launch: 4 kernels that clear 4 KiB 10.6 / 19
+// against 17.7 / 35, 5 13.3 / 21 against 18.0 / 35, but 6 20.6 / 23 against
+// 17.5 / 35, 12 40 / 79 against 26.5 / 38; 5 dots of 4096x4096 Q8_0 30.2 / 41
+// against 34.3 / 45.  A decode pass of 12 kernels (2048 columns) takes 51 / 76
+// against 57 / 65: faster in a row, but a decoder waits for every pass.  So the
+// line is where both are faster for the shortest kernels.
 namespace {
 struct graph_handle {
     hipGraphExec_t exec = nullptr;
-    hipGraph_t graph = nullptr;
-    std::vector<hipKernelNodeParams> chain;                       // arguments owned by graph
+    hipGraph_t graph = nullptr;                                   // owns the chain's arguments
+    int device = 0;
+    std::vector<hipKernelNodeParams> chain;
 };
-constexpr size_t GRAPH_CHAIN_MAX = 16;
+constexpr size_t GRAPH_CHAIN_MAX = 5;
 
 // the nodes of g in order, if they are one chain of at most GRAPH_CHAIN_MAX kernels
 bool kernel_chain(hipGraph_t g, std::vector<hipKernelNodeParams> & out) {
@@ -445,30 +484,55 @@ int flh_host_alloc(size_t bytes, void ** out) {
 }
 int flh_host_free(void * p) { return p ? hip_check(hipHostFree(p), "hipHostFree") : FLH_OK; }
 int flh_free(void * p) { return p ? hip_check(hipFree(p), "hipFree") : FLH_OK; }
+// (the turn is not held while the caller waits for the stream)
+static int copy_async(void * dst, const void * src, size_t n, hipMemcpyKind kind, void * stream, const char * what) {
+    const StreamTurn turn(stream);
+    return hip_check(hipMemcpyAsync(dst, src, n, kind, (hipStream_t)stream), what);
+}
 int flh_upload(void * dst, const void * src, size_t n, void * stream) {
-    if (int rc = hip_check(hipMemcpyAsync(dst, src, n, hipMemcpyHostToDevice, (hipStream_t)stream), "upload")) return rc;
+    if (int rc = copy_async(dst, src, n, hipMemcpyHostToDevice, stream, "upload")) return rc;
     return hip_check(hipStreamSynchronize((hipStream_t)stream), "upload sync");
 }
 int flh_download(void * dst, const void * src, size_t n, void * stream) {
-    if (int rc = hip_check(hipMemcpyAsync(dst, src, n, hipMemcpyDeviceToHost, (hipStream_t)stream), "download")) return rc;
+    if (int rc = copy_async(dst, src, n, hipMemcpyDeviceToHost, stream, "download")) return rc;
     return hip_check(hipStreamSynchronize((hipStream_t)stream), "download sync");
 }
 int flh_copy(void * dst, const void * src, size_t n, void * stream) {
-    return hip_check(hipMemcpyAsync(dst, src, n, hipMemcpyDeviceToDevice, (hipStream_t)stream), "copy");
+    return copy_async(dst, src, n, hipMemcpyDeviceToDevice, stream, "copy");
 }
-int flh_zero(void * dst, size_t n, void * stream) { return launch_zero(dst, n, (hipStream_t)stream); }
+int flh_zero(void * dst, size_t n, void * stream) {
+    const StreamTurn turn(stream);
+    return launch_zero(dst, n, (hipStream_t)stream);
+}
 
 // --------------------------------------------------------------- streams --
 int flh_stream_create(void ** out) {
     if (int rc = need_init()) return rc;
     if (!out) return set_error(FLH_ERR_ARG, "null out");
     hipStream_t s;
+    int dev = 0;
+    if (int rc = hip_check(hipGetDevice(&dev), "hipGetDevice")) return rc;
     if (int rc = hip_check(hipStreamCreateWithFlags(&s, hipStreamNonBlocking), "hipStreamCreate")) return rc;
+    auto st = std::make_shared<StreamTurn::State>();
+    st->device = dev;
+    {
+        StreamTurns & t = turns();
+        std::unique_lock<std::shared_mutex> l(t.m);
+        t.by_stream[(void *)s] = std::move(st);
+    }
     *out = (void *)s;
     return FLH_OK;
 }
 int flh_stream_sync(void * s) { return hip_check(hipStreamSynchronize((hipStream_t)s), "hipStreamSynchronize"); }
-int flh_stream_destroy(void * s) { return s ? hip_check(hipStreamDestroy((hipStream_t)s), "hipStreamDestroy") : FLH_OK; }
+int flh_stream_destroy(void * s) {
+    if (!s) return FLH_OK;
+    {
+        StreamTurns & t = turns();                                // before the handle can be another stream's
+        std::unique_lock<std::shared_mutex> l(t.m);
+        t.by_stream.erase(s);
+    }
+    return hip_check(hipStreamDestroy((hipStream_t)s), "hipStreamDestroy");
+}
 int flh_event_create(void ** out) {
     if (!out) return set_error(FLH_ERR_ARG, "null out");
     hipEvent_t e;
@@ -476,7 +540,10 @@ int flh_event_create(void ** out) {
     *out = (void *)e;
     return FLH_OK;
 }
-int flh_event_record(void * e, void * s) { return hip_check(hipEventRecord((hipEvent_t)e, (hipStream_t)s), "hipEventRecord"); }
+int flh_event_record(void * e, void * s) {
+    const StreamTurn turn(s);
+    return hip_check(hipEventRecord((hipEvent_t)e, (hipStream_t)s), "hipEventRecord");
+}
 int flh_event_elapsed_ms(void * a, void * b, float * ms) {
     if (!ms) return set_error(FLH_ERR_ARG, "null ms");
     if (int rc = hip_check(hipEventSynchronize((hipEvent_t)b), "hipEventSynchronize")) return rc;
@@ -487,10 +554,12 @@ int flh_event_destroy(void * e) { return e ? hip_check(hipEventDestroy((hipEvent
 // ---------------------------------------------------------------- graphs --
 int flh_graph_capture_begin(void * stream) {
     if (int rc = need_init()) return rc;
+    const StreamTurn turn(stream);
     return hip_check(hipStreamBeginCapture((hipStream_t)stream, hipStreamCaptureModeThreadLocal),
                      "hipStreamBeginCapture");
 }
 int flh_graph_capture_end(void * stream, void ** graph_exec) {
+    const StreamTurn turn(stream);
     hipGraph_t g = nullptr;
     // (with a null graph_exec the capture still ends, so the stream is usable)
     if (int rc = hip_check(hipStreamEndCapture((hipStream_t)stream, &g), "hipStreamEndCapture")) return rc;
@@ -499,15 +568,18 @@ int flh_graph_capture_end(void * stream, void ** graph_exec) {
         return set_error(FLH_ERR_ARG, "null graph_exec");
     }
     graph_handle * h = new graph_handle();
-    if (kernel_chain(g, h->chain)) {
-        h->graph = g;                                             // holds the arguments
-    } else {
-        const int rc = hip_check(hipGraphInstantiate(&h->exec, g, nullptr, nullptr, 0), "hipGraphInstantiate");
+    int rc = hip_check(hipGetDevice(&h->device), "hipGetDevice");
+    if (!rc) rc = hip_check(hipGraphInstantiate(&h->exec, g, nullptr, nullptr, 0), "hipGraphInstantiate");
+    if (rc) {
         (void)hipGraphDestroy(g);
-        if (rc) {
-            delete h;
-            return rc;
-        }
+        delete h;
+        return rc;
+    }
+    if (kernel_chain(g, h->chain)) {
+        h->graph = g;
+    } else {
+        h->chain.clear();
+        (void)hipGraphDestroy(g);
     }
     *graph_exec = (void *)h;
     return FLH_OK;
@@ -515,11 +587,16 @@ int flh_graph_capture_end(void * stream, void ** graph_exec) {
 int flh_graph_launch(void * ge, void * stream) {
     const graph_handle * h = (const graph_handle *)ge;
     if (!h) return set_error(FLH_ERR_ARG, "null graph");
-    if (h->exec) return hip_check(hipGraphLaunch(h->exec, (hipStream_t)stream), "hipGraphLaunch");
-    // one replay at a time: threads that replay onto one stream get whole graphs
-    // in some order, as from the runtime's launch, not their kernels interleaved
-    static std::mutex whole;
-    std::lock_guard<std::mutex> lock(whole);
+    // A replay is one operation of its stream.  The runtime's launch is one by
+    // itself.  A chain is one because its thread has the stream to itself
+    // meanwhile (every entry point that issues work takes part in that), so it is
+    // only for a stream made here, on the device in force and not being captured.
+    const StreamTurn turn(stream, !h->chain.empty());
+    int dev = -1;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (h->chain.empty() || turn.device() != h->device || hipGetDevice(&dev) != hipSuccess || dev != h->device ||
+        hipStreamIsCapturing((hipStream_t)stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone)
+        return hip_check(hipGraphLaunch(h->exec, (hipStream_t)stream), "hipGraphLaunch");
     for (const hipKernelNodeParams & k : h->chain)
         if (int rc = hip_check(hipLaunchKernel(k.func, k.gridDim, k.blockDim, k.kernelParams, k.sharedMemBytes,
                                                (hipStream_t)stream), "graph kernel launch")) return rc;
@@ -528,8 +605,11 @@ int flh_graph_launch(void * ge, void * stream) {
 int flh_graph_destroy(void * ge) {
     graph_handle * h = (graph_handle *)ge;
     if (!h) return FLH_OK;
-    const int rc = h->exec ? hip_check(hipGraphExecDestroy(h->exec), "hipGraphExecDestroy")
-                           : hip_check(hipGraphDestroy(h->graph), "hipGraphDestroy");
+    int rc = hip_check(hipGraphExecDestroy(h->exec), "hipGraphExecDestroy");
+    if (h->graph) {
+        const int rc2 = hip_check(hipGraphDestroy(h->graph), "hipGraphDestroy");
+        if (!rc) rc = rc2;
+    }
     delete h;
     return rc;
 }
@@ -537,6 +617,7 @@ int flh_graph_destroy(void * ge) {
 // ------------------------------------------------------------------- ops --
 int flh_act_q8(float * x, void * y_q81, uint32_t cols, uint32_t nx, uint32_t xstride, void * stream) {
     if (int rc = need_init()) return rc;
+    const StreamTurn turn(stream);
     if (nx == 0) nx = 1;
     if (!x || ((uintptr_t)x & 15) || (nx > 1 && (xstride & 3)))
         return set_error(FLH_ERR_ARG, "act_q8: x must be non-null and 16-byte aligned, xstride a multiple of 4");
@@ -552,6 +633,7 @@ int flh_stream_dot(int fmt, const void * w, uint64_t w_bytes, uint32_t rows, uin
     if (nx == 0) nx = 1;
     if (int rc = validate_dot(fmt, w, w_bytes, rows, cols, x, y, nx, id_slot, estride, ystride)) return rc;
     if (int rc = need_init()) return rc;
+    const StreamTurn turn(stream);
     DotArgs a{(const uint8_t *)w, id_slot, estride, x, y, rows, cols, nx, xstride, ystride};
     return dispatch_dot(fmt, a, fast, i8_mask, i8k_mask, (hipStream_t)stream);
 }
@@ -566,6 +648,7 @@ int flh_act_q8_stream_dot(int fmt, const void * w, uint64_t w_bytes, uint32_t ro
         return set_error(FLH_ERR_ARG, "act_q8: x must be 16-byte aligned, xstride a multiple of 4");
     if (int rc = validate_xstride(cols, nx, xstride)) return rc;
     if (int rc = need_init()) return rc;
+    const StreamTurn turn(stream);
     hipStream_t s = (hipStream_t)stream;
     DotArgs a{(const uint8_t *)w, id_slot, estride, x, y, rows, cols, nx, xstride, ystride};
     // Fused when every workgroup re-reading the fp32 column is cheaper than a
@@ -605,6 +688,7 @@ int flh_rmsnorm_stream_dot(int fmt, const void * w, uint64_t w_bytes, uint32_t r
         return set_error(FLH_ERR_ARG, "rmsnorm dot: x, wnorm, xn non-null and 16-byte aligned");
     if (cols % 256) return set_error(FLH_ERR_ARG, "rmsnorm dot: cols must be a multiple of 256 (the q8_K appendix)");
     if (int rc = need_init()) return rc;
+    const StreamTurn turn(stream);
     const float * xe = x + cols;
     const float * ye = (const float *)((const uint8_t *)xn + x_alloc_bytes(cols));
     if (x < ye && xn < xe) return set_error(FLH_ERR_ARG, "rmsnorm dot: xn overlaps x");
@@ -614,6 +698,7 @@ int flh_rmsnorm_stream_dot(int fmt, const void * w, uint64_t w_bytes, uint32_t r
 
 int flh_dequant(int fmt, const void * w, uint32_t rows, uint32_t cols, float * out, void * stream) {
     if (int rc = need_init()) return rc;
+    const StreamTurn turn(stream);
     if (cols % blk_elems(fmt)) return set_error(FLH_ERR_ARG, "dequant: cols not a multiple of the block size");
     return launch_dequant(fmt, (const uint8_t *)w, rows, cols, out, (hipStream_t)stream);
 }
@@ -622,6 +707,7 @@ int flh_exec_tasks(const flh_task * t, uint32_t n, int fast, uint32_t i8_mask, u
                    void * stream) {
     if (int rc = validate_table(t, n)) return rc;
     if (int rc = need_init()) return rc;
+    const StreamTurn turn(stream);
     hipStream_t s = (hipStream_t)stream;
     for (uint32_t i = 0; i < n; ++i) {
         const flh_task & k = t[i];
@@ -723,6 +809,7 @@ int flh_moe_dot(int fmt, const void * w, uint64_t estride, uint32_t rows, uint32
                 const float * x, uint32_t xstride, uint32_t x_per_slot, float * y, uint32_t ystride,
                 void * stream) {
     if (int rc = need_init()) return rc;
+    const StreamTurn turn(stream);
     if (fmt < FLH_FMT_Q8_0 || fmt > FLH_FMT_IQ3_XXS)
         return set_error(FLH_ERR_UNSUPPORTED, "moe_dot: quantized weight formats only");
     if (cols % 256 || cols == 0) return set_error(FLH_ERR_ARG, "moe_dot: cols not a positive multiple of 256");
@@ -741,6 +828,7 @@ int flh_router_moe_dot(int fmt, const void * w, uint64_t estride, uint32_t rows,
                        float scale, uint32_t * ids, float * gates, const float * x, uint32_t xstride,
                        uint32_t x_per_slot, float * y, uint32_t ystride, void * stream) {
     if (int rc = need_init()) return rc;
+    const StreamTurn turn(stream);
     if (fmt < FLH_FMT_Q8_0 || fmt > FLH_FMT_IQ3_XXS)
         return set_error(FLH_ERR_UNSUPPORTED, "router_moe_dot: quantized weight formats only");
     const bool kf = fmt == FLH_FMT_Q4_K || fmt == FLH_FMT_Q6_K;
@@ -775,16 +863,19 @@ int flh_router_moe_dot(int fmt, const void * w, uint64_t estride, uint32_t rows,
 int flh_router_sel(const float * logits, uint32_t ntok, uint32_t n_expert, uint32_t top_k, uint32_t norm,
                    float scale, uint32_t * ids, float * gates, void * stream) {
     if (int rc = need_init()) return rc;
+    const StreamTurn turn(stream);
     return launch_router_sel(logits, ntok, n_expert, top_k, norm, scale, ids, gates, (hipStream_t)stream);
 }
 int flh_silu_mul(const float * gate, const float * up, float * h, uint32_t n, uint32_t ncol,
                  uint32_t gstride, uint32_t hstride, void * stream) {
     if (int rc = need_init()) return rc;
+    const StreamTurn turn(stream);
     return launch_silu_mul(gate, up, h, n, ncol, gstride, hstride, (hipStream_t)stream);
 }
 int flh_rmsnorm_act_q8(const float * x, const float * wnorm, float * y, uint32_t n, float eps, int write_app,
                        void * stream) {
     if (int rc = need_init()) return rc;
+    const StreamTurn turn(stream);
     if (!x || !wnorm || !y || ((uintptr_t)x & 3) || ((uintptr_t)wnorm & 3) || ((uintptr_t)y & (write_app ? 15 : 3)))
         return set_error(FLH_ERR_ARG, "rmsnorm: x, wnorm, y non-null and aligned (y 16 bytes with ACT_Q8)");
     return launch_rmsnorm_act_q8(x, wnorm, y, n, eps, write_app != 0, (hipStream_t)stream);
@@ -793,6 +884,7 @@ int flh_rmsnorm_act_q8(const float * x, const float * wnorm, float * y, uint32_t
 int flh_silu_mul_act_q8(const float * gate, const float * up, float * h, uint32_t n, uint32_t ncol,
                         uint32_t gstride, uint32_t hstride, void * stream) {
     if (int rc = need_init()) return rc;
+    const StreamTurn turn(stream);
     if (!gate || !up || !h || ((uintptr_t)h & 15) || (ncol > 1 && (hstride & 3)))
         return set_error(FLH_ERR_ARG, "silu_mul_act_q8: h must be 16-byte aligned, hstride a multiple of 4");
     return launch_silu_act_q8(gate, up, h, n, ncol, gstride, hstride, (hipStream_t)stream);
@@ -801,6 +893,7 @@ int flh_wmerge(const float * parts, const float * gates, const float * add1, con
                float scale, uint32_t n_parts, uint32_t n, uint32_t n_full, uint32_t ncol, uint32_t pstride,
                uint32_t ystride, void * stream) {
     if (int rc = need_init()) return rc;
+    const StreamTurn turn(stream);
     return launch_wmerge(parts, gates, add1, add2, y, scale, n_parts, n, n_full, ncol, pstride, ystride,
                          (hipStream_t)stream);
 }
@@ -809,10 +902,12 @@ int flh_wmerge(const float * parts, const float * gates, const float * add1, con
 int flh_fill_normal(float * dst, size_t n, uint64_t seed, float mean, float stddev, float outlier_frac,
                     float outlier_scale, void * stream) {
     if (int rc = need_init()) return rc;
+    const StreamTurn turn(stream);
     return launch_fill_normal(dst, n, seed, mean, stddev, outlier_frac, outlier_scale, (hipStream_t)stream);
 }
 int flh_quantize(int fmt, const float * src, uint32_t rows, uint32_t cols, void * dst, void * stream) {
     if (int rc = need_init()) return rc;
+    const StreamTurn turn(stream);
     return launch_quantize_weights(fmt, src, rows, cols, (uint8_t *)dst, (hipStream_t)stream);
 }
 int flh_quantize_host(int fmt, const float * src, uint32_t rows, uint32_t cols, void * dst) {

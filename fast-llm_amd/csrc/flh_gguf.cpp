@@ -394,6 +394,7 @@ int staged_h2d(uint8_t * dst, const uint8_t * src, size_t n, hipStream_t s) {
         if (g_stage.used[k])
             if (int rc = hip_check(hipEventSynchronize(g_stage.done[k]), "gguf staging wait")) return rc;
         parallel_copy(g_stage.buf[k], src + done, len);
+        const flh::StreamTurn turn((void *)s);
         if (int rc = hip_check(hipMemcpyAsync(dst + done, g_stage.buf[k], len, hipMemcpyHostToDevice, s),
                                "gguf upload hipMemcpyAsync"))
             return rc;

@@ -5,8 +5,36 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include <stddef.h>
+#include <memory>
+#include <mutex>
+#include <shared_mutex>
 
 namespace flh {
+
+// Held by an entry point while it issues work on a stream.  A replay that is
+// launched kernel by kernel holds it whole: it waits for the calls that are
+// issuing on that stream, and later ones wait for it, so no other thread's work
+// falls between its kernels.  The other calls do not exclude each other, and
+// streams never wait for one another (a turn is found by the stream's handle).
+// A stream that was not made by flh_stream_create has none (device() is -1),
+// and nothing to wait for: no replay on it is more than one runtime call.
+class StreamTurn {
+public:
+    struct State {
+        std::mutex gate;
+        std::shared_mutex m;
+        int device = -1;
+    };
+    explicit StreamTurn(void * stream, bool whole = false);
+    ~StreamTurn();
+    StreamTurn(const StreamTurn &) = delete;
+    StreamTurn & operator=(const StreamTurn &) = delete;
+    int device() const { return st_ ? st_->device : -1; }
+
+private:
+    std::shared_ptr<State> st_;
+    const bool whole_;
+};
 
 // One STREAM_DOT launch: y[p*ystride + r] += dot(W[r], x + p*xstride),
 // r < rows, p < nx.  W = w (+ *id_slot * estride when id_slot != nullptr,

@@ -178,8 +178,16 @@ int flh_event_destroy(void * event);
  * persistent-kernel launch amortisation, src/runtime/gpu_exec.cu:156-344,
  * for a frozen graph: capture once, replay per token).  Every kernel of
  * this library is capture-safe (no hipMemsetAsync, no host syncs).  The
- * handle is this library's own (a short chain of kernels is replayed kernel by
- * kernel, anything else as the runtime's graph): launch and destroy it here. */
+ * handle is this library's own: launch and destroy it here.
+ *
+ * A replay is one operation of its stream: work that other threads issue there
+ * through this library comes before or after all of it.  On a stream of
+ * flh_stream_create a chain of at most 5 kernels is replayed kernel by kernel
+ * (less idle time on the device, less of the caller's time); what other code
+ * issues there directly (a HIP call on the handle) from another thread at the
+ * same time may then fall between two of the kernels, and a replay that fails
+ * may have run in part.  On any other stream, and for any other graph, a replay
+ * is the runtime's own graph launch. */
 int flh_graph_capture_begin(void * stream);
 int flh_graph_capture_end(void * stream, void ** graph_exec);
 int flh_graph_launch(void * graph_exec, void * stream);

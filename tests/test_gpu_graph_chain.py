@@ -1,5 +1,5 @@
 """Captured graphs: short chains of kernels (launched one by one on replay), at
-and past the 16-kernel line, and a capture with a copy node (the runtime's
+and past the 5-kernel line, and a capture with a copy node (the runtime's
 form).  Every replay equals the eager result, with eager work, a change of the
 inputs and synchronizations between the replays, on the captured stream and on
 another one."""
@@ -13,10 +13,11 @@ from test_gpu_parity import bits, say
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("layers,copy", [(0, False), (1, False), (5, False), (5, True), (6, False), (9, False)])
-def test_replays_equal_eager(flh, gpu, layers, copy):
-    """1 + 3 * layers launches (and a copy): zero, then ACT_Q8, dot, dot."""
-    say("graph chain", layers, copy)
+@pytest.mark.parametrize("layers,more,copy", [(0, 0, False), (1, 0, False), (1, 1, False), (1, 2, False), (2, 0, False),
+                                              (1, 0, True), (5, 0, False), (5, 0, True), (6, 0, False), (9, 0, False)])
+def test_replays_equal_eager(flh, gpu, layers, more, copy):
+    """1 + 3 * layers + more launches (and a copy): zero, then ACT_Q8, dot, dot."""
+    say("graph chain", layers, more, copy)
     rows, cols = 96, 512
     rng = np.random.default_rng(layers)
     st = col_stride_floats(cols)
@@ -32,6 +33,8 @@ def test_replays_equal_eager(flh, gpu, layers, copy):
             flh.act_q8(dx, cols, s)
             for k in range(2):
                 flh.stream_dot(Q4_K, dw[l], rows, cols, dx, dy.ptr + 4 * rows * (2 * l + k), s)
+        for _ in range(more):
+            flh.stream_dot(Q4_K, dw[0], rows, cols, dx, dy, s)
         if copy:
             flh.copy(dz, dy, 4 * rows, s)
 
