@@ -313,24 +313,36 @@ __global__ __launch_bounds__(256) void k_dequant(const uint8_t * __restrict__ w,
         }
 }
 
+// A launch holds fewer than 2^32 threads, so 2^24 workgroups (2^35 outputs) and
+// more go in several.
+template <int FMT>
+static int deq_go(const uint8_t * w, uint64_t n32, float * out, hipStream_t s) {
+    constexpr uint64_t B32 = 8 * 4 * DEQ_UN, MOST = (1ull << 24) - 1;   // 32-weight blocks per workgroup; workgroups
+    constexpr uint64_t BB = FMT == FMT_Q8_0 ? 34 : FMT == FMT_Q5_0 ? 22 : 0;   // bytes of a block
+    constexpr uint64_t UB = BB ? 8 * BB : FMT == FMT_Q4_K ? 144 : FMT == FMT_Q6_K ? 210 : iq_block_bytes(FMT);   // of a unit
+    while (n32) {
+        const uint64_t nwg = min((n32 + B32 - 1) / B32, MOST), n = min(n32, nwg * B32);
+        hipLaunchKernelGGL(k_dequant<FMT>, dim3((uint32_t)nwg), dim3(256), 0, s, w, n, out);
+        if (int rc = hip_check(hipGetLastError(), "k_dequant launch")) return rc;
+        n32 -= n;
+        w += n / 8 * UB;                                          // (n is a multiple of 8 unless it is the last)
+        out += n * 32;
+    }
+    return FLH_OK;
+}
+
 int launch_dequant(int fmt, const uint8_t * w, uint32_t rows, uint32_t cols,
                    float * out, hipStream_t s) {
-    if (fmt < FMT_Q8_0 || fmt > FMT_IQ3_XXS)
-        return set_error(FLH_ERR_UNSUPPORTED, "dequant: format not supported");
     const uint64_t n32 = (uint64_t)rows * (cols / 32);
-    if (n32 == 0) return FLH_OK;
-    const uint64_t nwg = (n32 + 8 * 4 * DEQ_UN - 1) / (8 * 4 * DEQ_UN);
-    if (nwg > 0x7FFFFFFFull) return set_error(FLH_ERR_UNSUPPORTED, "dequant: more than 2^43 outputs");
-    const dim3 g((uint32_t)nwg), b(256);
     switch (fmt) {
-        case FMT_Q8_0: hipLaunchKernelGGL(k_dequant<FMT_Q8_0>, g, b, 0, s, w, n32, out); break;
-        case FMT_Q5_0: hipLaunchKernelGGL(k_dequant<FMT_Q5_0>, g, b, 0, s, w, n32, out); break;
-        case FMT_Q4_K: hipLaunchKernelGGL(k_dequant<FMT_Q4_K>, g, b, 0, s, w, n32, out); break;
-        case FMT_Q6_K: hipLaunchKernelGGL(k_dequant<FMT_Q6_K>, g, b, 0, s, w, n32, out); break;
-        case FMT_IQ2_XXS: hipLaunchKernelGGL(k_dequant<FMT_IQ2_XXS>, g, b, 0, s, w, n32, out); break;
-        default: hipLaunchKernelGGL(k_dequant<FMT_IQ3_XXS>, g, b, 0, s, w, n32, out); break;
+        case FMT_Q8_0: return deq_go<FMT_Q8_0>(w, n32, out, s);
+        case FMT_Q5_0: return deq_go<FMT_Q5_0>(w, n32, out, s);
+        case FMT_Q4_K: return deq_go<FMT_Q4_K>(w, n32, out, s);
+        case FMT_Q6_K: return deq_go<FMT_Q6_K>(w, n32, out, s);
+        case FMT_IQ2_XXS: return deq_go<FMT_IQ2_XXS>(w, n32, out, s);
+        case FMT_IQ3_XXS: return deq_go<FMT_IQ3_XXS>(w, n32, out, s);
+        default: return set_error(FLH_ERR_UNSUPPORTED, "dequant: format not supported");
     }
-    return hip_check(hipGetLastError(), "k_dequant launch");
 }
 
 }  // namespace flh
