@@ -89,6 +89,12 @@ template <int FMT, int NC> struct CwPlan {
     static constexpr uint32_t NX = KF ? 0 : NC * CW<FMT>::CU / 8, NT = NW + NA + NX;
     static constexpr uint32_t XOFF = (NW + NA) * 1024, STG = XOFF + NX * 256;
 };
+// A chunk of `units` 256-column units of a column is staged in 16-byte pieces
+// that end where its bytes end, and so begin up to 12 bytes below it (q8_K: 292
+// bytes a unit; a whole chunk is whole pieces): nothing is read past the column,
+// wherever it lies (K formats: at any 4-byte boundary, where 16-byte
+// direct-to-LDS loads are as fast).
+template <int FMT> __device__ __forceinline__ uint32_t cw_xshift(uint32_t units) { return (0u - units * CW<FMT>::UA) & 15u; }
 constexpr uint32_t CW_WAVES = 5;                                  // four consumers and the producer
 constexpr uint32_t CW_ZERO = 320;                                 // zero bytes that off-diagonal lanes read
 // LDS: [D][STG] ring | [4][16][16] sums | zeros | codebook (2 KiB), sign masks (1 KiB)
@@ -210,7 +216,7 @@ __device__ __forceinline__ void cw_produce(const uint8_t * __restrict__ w, uint3
         }
         uint8_t * stage = sm + (size_t)qslot * STG;
         const uint8_t * wb = w + (size_t)row0 * RB + (size_t)qc * CB;
-        const uint8_t * xb = x0 + (size_t)qc * CA;
+        const uint8_t * xb = x0 + (size_t)qc * CA - (qc + 1 < nch ? 0u : cw_xshift<FMT>(lastu));
         if (qc + 1 < nch || lastu == P::CU || cw_gran(FMT)) {
             const uint32_t sh = (uint32_t)(uintptr_t)wb & 15u;    // the chunk's offset in its granule
             const bool part = qc + 1 == nch && lastu < P::CU;     // (these formats only)
@@ -320,9 +326,9 @@ __device__ __forceinline__ void cw_consume(const uint8_t * __restrict__ w, uint3
         for (uint32_t c = 0; c < nch; ++c) {
             lds_barrier();
             const uint32_t st = lds_off(sm + (size_t)slot * STG);
-            const uint32_t xs = st + 1024 * L::NW, xt = st + L::XOFF;   // the columns, the table
-            slot = slot + 1 == (uint32_t)D ? 0 : slot + 1;
             const uint32_t units = c + 1 == nch ? lastu : P::CU;
+            const uint32_t xs = st + 1024 * L::NW + cw_xshift<FMT>(units), xt = st + L::XOFF;   // the columns, the table
+            slot = slot + 1 == (uint32_t)D ? 0 : slot + 1;
             if constexpr (cw_iq(FMT)) {
                 // lane (r, j): blocks b = 16 h + 4 j + k of row r, group 4 (j & 1) + k
                 // of superblock 2 h + j / 2; the row's chunk starts sh bytes into its window
@@ -657,7 +663,8 @@ __global__ __launch_bounds__(64 * CW_WAVES, 4) void k_moe_cw(MoeArgs a) {
 // ----------------------------------------------------------------- launch --
 static bool cw_takes(int fmt, const void * w, uint64_t estride, const void * x, uint32_t xstride, uint32_t ncol,
                      uint32_t cols) {
-    if (cols == 0 || (cols & 255) || ((uintptr_t)x & 15) || (xstride & 3)) return false;
+    if (cols == 0 || (cols & 255) || ((uintptr_t)x & 3)) return false;
+    if (fmt != FMT_Q4_K && fmt != FMT_Q6_K && (((uintptr_t)x & 15) || (xstride & 3))) return false;
     // 32-bit lane offsets
     if ((uint64_t)ncol * xstride * 4 + x_alloc_bytes(cols) >= (1ull << 32) || 16ull * cols * 2 >= (1ull << 32)) return false;
     // Q6_K and IQ rows are placed from their own 16-byte boundaries; the others' rows
