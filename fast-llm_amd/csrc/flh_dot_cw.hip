@@ -693,45 +693,71 @@ template <int FMT> static int cw_launch(const DotArgs & a, hipStream_t s) {
 }
 
 // Whether a matrix with nx columns is faster here than on the format's other
-// kernel (us here / there):
-//  * Q4_K against k_dot_mfma, whose tiles are 16 x 144-byte pieces but which
-//    stages the columns once per workgroup: 4 columns 14336x4096 9.6 / 10.6,
-//    4096x14336 9.2 / 11.7; 8 columns 6144x4096 6.6 / 7.9, 4096x14336 11.5 / 14.6,
-//    14336x4096 10.8 / 11.6, 28672x4096 17.1 / 17.9; 16 columns 4352x1792 6.2 /
-//    6.8, 6144x4096 8.4 / 9.6, 9216x3840 13.2 / 13.0, 14336x4096 14.3 / 14.5, but
-//    28672x4096 23.1 / 21.7 (the columns are as many bytes as the weights), and
-//    where that kernel needs several passes 27648x5120 38 / 46, 8192x8192 20 / 25.
-//  * Q6_K against the streaming kernel: 2 columns 14336x4096 14.5 / 12.1,
-//    4096^2 7.4 / 6.5, 4096x14336 15.7 / 16.5; 3 columns 14336x4096 14.5 / 16.2,
-//    6144x4096 9.2 / 9.1; 8 columns 14336x4096 15.7 / 21.7, 4096x14336 15.9 / 40;
-//    a 128256x4096 vocabulary with 3 / 8 / 16 columns 97 / 95 / 122 against
-//    101 / 102 / 154 (the last two on a Q6_K matrix-core kernel of their own).
+// kernel (us here / there, medians of back-to-back launches over matrices in
+// HBM).  A workgroup takes whole 16-row tiles of whole rows: with half as many
+// tiles as CUs, or fewer, a launch takes as long as one tile however few there
+// are, about 4.3 + 0.75 us per chunk of a row, and kernels that split the rows
+// further are faster on all but short rows.  Elsewhere:
+//  * Q4_K against k_dot_mfma (k_dot_kstream with 2 columns of up to 4096), whose
+//    tiles are 16 x 144-byte pieces but which stages the columns once per
+//    workgroup.  4 columns 14336x4096 9.7 / 10.3, 4096x14336 9.4 / 11.3; 8
+//    columns 6144x3840 7.4 / 8.1, 14336x4096 11.3 / 11.8, 8192x14336 16.6 / 26.9;
+//    16 columns 14336x4096 14.6 / 14.7, 28672x4096 21.8 / 21.7 (the columns are as
+//    many bytes as the weights), where that kernel takes several passes
+//    28672x5120 27.8 / 46.2.  Rows that end in part of a chunk cost a whole one:
+//    8 columns 28672x2304 14.8 / 13.4, 28672x3840 18.1 / 17.4 (20480x2816 11.9 /
+//    11.8), 16 columns 9216x3328 13.2 / 12.6 (6144x3328 8.9 / 9.5).  Few long rows:
+//    5 columns 512x14336 11.6 / 11.3; 2 columns 100x4096 4.9 / 4.4.
+//  * Q6_K against the streaming kernel.  2 columns 4096x14336 15.6 / 16.2,
+//    3072x14336 15.4 / 14.0, 14336x4096 14.5 / 12.1; 4 columns 4096x4096 7.8 / 8.0,
+//    2048x4096 7.5 / 6.8, 1024x8192 10.4 / 7.0, 1024x2048 5.0 / 5.9; 8 columns
+//    2048x4096 7.5 / 8.1, 1024x4096 7.5 / 6.8, 1024x8192 10.6 / 9.9, 512x14336 15.0
+//    / 16.5, 14336x4096 15.6 / 33.
 //  * Q8_0 and Q5_0 against k_dot_sbl_nx (rows of up to 8192 columns) and the
-//    register kernel: 2 columns Q8_0 14336x4096 15.3 / 14.4, 4096x14336 14.8 /
-//    20.6, Q5_0 14336x4096 12.1 / 14.0; 4 columns 15.5 / 18.5, 12.4 / 17.1,
-//    4096x14336 15 / 46; 16 columns 14336x4096 22.7 / 52, 4096x14336 23 / 149.
-//    A few long rows leave most of the chip idle here: Q8_0 1024x2816 with 2 / 4
-//    columns 5.5 / 4.6 and 5.5 / 5.2.  One column against k_dot_sbl: rows wider
-//    than its one pass per lane group holds well, Q8_0 4096x14336 14.7 / 18.3,
-//    8192x8192 14.7 / 17.0, Q5_0 27648x5120 22.6 / 32.8; not 14336x4096 15.2 / 13.4,
+//    register kernel.  2 columns Q8_0 14336x4096 15.3 / 14.4, 4096x8192 9.9 / 11.5,
+//    2048x8192 9.4 / 8.1, 4096x14336 14.2 / 20.1, Q5_0 14336x4096 12.3 / 14.2,
+//    2048x4096 6.5 / 5.8; 4 columns Q8_0 1024x4096 6.4 / 6.4, 14336x4096 15.7 /
+//    18.1; 5 columns Q5_0 512x8192 11.3 / 10.1 (8 columns 11.4 / 11.7), Q8_0 256x6144
+//    8.9 / 8.1; 16 columns 14336x4096 20 / 52.  One column against k_dot_sbl: rows
+//    wider than its one pass per lane group holds well, Q8_0 4096x14336 14.3 / 18.6,
+//    8192x8192 14.1 / 17.1, Q5_0 8192x14336 17.8 / 29.6; not 14336x4096 15.2 / 13.4,
 //    2048x5632 7.6 / 6.3.
 //  * IQ2_XXS and IQ3_XXS against k_dot_sbl_nx (rows of up to 8192 columns, a
-//    multiple of 2048), k_dot_sbl (one column) and the register kernel: IQ2_XXS
-//    14336x4096 with 2 / 4 / 8 / 16 columns 13.8 / 12.5, 13.7 / 14.8, 18.2 / 21.5,
-//    26.7 / 42.5; 28672x4096 with 2 20.9 / 22.8; 4096x14336 with 2 / 8 16.2 / 26.8,
-//    20.4 / 61.6; IQ3_XXS 14336x4096 with 2 / 4 16.2 / 14.6, 16.1 / 16.9.  Rows
-//    that are no multiple of 2048 columns, 3840x3840 with 1 / 2 / 16: 6.5 / 7.7,
-//    6.5 / 8.7, 10.2 / 44; one column of few rows, 1024x2816: 5.4 / 5.1.
+//    multiple of 2048), k_dot_sbl (one column) and the register kernel.  2 columns
+//    IQ2_XXS 14336x4096 13.8 / 12.5, 28672x4096 21.3 / 23.2, IQ3_XXS 28672x2048 14.7 /
+//    13.8; 4 columns IQ2_XXS 4096x4096 7.3 / 7.7, 2048x4096 7.2 / 6.2, 1024x8192
+//    10.5 / 7.0; 8 columns 2048x4096 8.9 / 8.3, 2048x8192 12.9 / 14.0 (5 columns 13.0
+//    / 12.2), 1024x8192 12.9 / 11.9; 16 columns 14336x4096 25.7 / 42.6.  Other row
+//    lengths: 2 columns 1024x2816 5.9 / 5.8, 2048x2816 6.3 / 7.9, 1024x14336 15.8 /
+//    14.8; 4 columns 256x1792 IQ3_XXS 4.9 / 4.5, 512x2816 5.8 / 5.7; 3840x3840 with 1
+//    / 16 6.5 / 7.7, 10.2 / 44; one column of few rows, 1024x2816: 5.4 / 5.1.
 static bool cw_wins(int fmt, uint32_t rows, uint32_t cols, uint32_t nx) {
     const uint32_t T = (rows + 15) / 16, cus = (uint32_t)num_cus();
-    if (fmt == FMT_Q4_K) return nx <= 8 || rows <= 16384 || cols > 4096;
-    if (fmt == FMT_Q6_K) return nx > 2 || cols > 8192;
+    const bool half = 2 * T <= cus, quarter = 4 * T <= cus, sixteenth = 16 * T <= cus;   // of the chip, at most
+    if (fmt == FMT_Q4_K) {
+        const bool part = (cols & 1023) && cols > 1024;
+        if (nx > 8) return cols > 4096 || rows <= (part ? 8192u : 16384u);
+        if (nx > 4) return !(part && rows > 20480) && !(half && cols > 8192);
+        return !(nx == 2 && sixteenth && cols > 2048 && cols <= 4096);
+    }
+    if (fmt == FMT_Q6_K) {
+        if (nx == 2) return cols > 8192 && T >= cus;
+        if (nx <= 4) return !(half && cols > 2048);
+        return nx > 8 || !((cols <= 8192 ? quarter : sixteenth) && cols > 2816);
+    }
     if (cw_iq(fmt)) {
+        const bool sbl = !(cols & 2047) && cols <= 8192;
         if (nx == 1) return cols > 16128 || ((cols & 2047) && rows >= 2048);
-        return nx > 2 || cols > 8192 || (cols & 2047) || rows > 16384;
+        if (nx == 2) return sbl ? rows > 16384 && cols > 2048 : !(quarter && cols > 1024);
+        if (nx <= 4 && sbl) return !(half && cols > 2048);
+        if (nx <= 4) return !(sixteenth && cols > 1024) && !((cols > 8192 ? quarter : 5 * T <= cus) && cols > 2048);
+        return nx > 8 || !(sbl && cols > 2048 && (cols <= 6144 || nx <= 6 ? half : quarter));
     }
     if (nx == 1) return cols > 4096 && T >= cus;
-    if (nx <= 4 && 4 * T <= cus && cols > 2048) return false;
+    if (nx == 2 && half && cols > 2048 && cols <= 8192) return false;
+    if (nx <= 4 && quarter && cols > 2048) return false;
+    if (nx > 4 && nx <= 8 && sixteenth && cols > 4096 && cols <= 6144) return false;
+    if (fmt == FMT_Q5_0 && (nx == 5 || nx == 6) && quarter && cols > 4096 && cols <= 8192) return false;
     return nx > 2 || fmt == FMT_Q5_0 || cols > 4096;
 }
 static bool cw_on(int fmt) {
