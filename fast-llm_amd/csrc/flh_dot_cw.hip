@@ -792,8 +792,45 @@ template <int FMT> static int cw_moe(const MoeArgs & a, hipStream_t s) {
     hipLaunchKernelGGL((k_moe_cw<FMT>), dim3(wgs), dim3(64 * CW_WAVES), smb, s, a);
     return hip_check(hipGetLastError(), "k_moe_cw launch");
 }
-int launch_moe_cw(int fmt, const MoeArgs & a, hipStream_t s) {
-    if (!cw_on(fmt)) return FLH_ERR_UNSUPPORTED;
+// Whether grouped experts of several tokens are faster here than on the format's
+// other kernel, which reads an expert once for each of its pairs (us here /
+// there; 8 experts take 2 of 8, 128 take 8 of 128).  So the line is a number of
+// pairs per expert that some token takes, on average:
+//  * Q8_0, Q5_0 and the IQ formats against the routed k_dot_sbl (rows of up to
+//    8192 columns).  That launch is about one workgroup per CU and as many for
+//    every pair, so where the pairs do not divide the CUs some wait for a second turn:
+//    Q8_0 3072x2048, 64 experts, 6 of them a token, 2 / 4 tokens 18.5 / 26.4, 29.8 /
+//    47.7.  Elsewhere Q8_0 256x1024 of 8 with 2 / 16 tokens 5.6 / 4.5, 6.3 / 4.9, of
+//    128 with 8 / 16 8.0 / 6.7, 10.2 / 9.6 (Q5_0 9.6 / 9.3); 1024x2048 of 8 with 4
+//    / 8 7.4 / 6.3, 7.7 / 8.5, of 128 with 8 / 16 26.7 / 23.2, 38.2 / 43.2; 3072x2048
+//    of 8 with 4 / 8 11.5 / 10.8, 13.5 / 18.0; 4096x4096 of 8 with 2 / 4 15.3 / 15.2,
+//    22.9 / 25.4 (Q5_0 13.1 / 14.1 with 2), of 128 with 4 / 8 92 / 89, 164 / 174;
+//    IQ2_XXS 3072x2048 of 8 with 4 / 8 12.3 / 10.7, 13.5 / 16.5, of 128 with 8 / 16
+//    62 / 51, 98 / 97; 4096x4096 of 8 with 4 24.1 / 22.2, of 128 with 8 / 16 151 /
+//    141, 249 / 275; 14336x4096 of 8 with 2 / 4 39 / 35, 56 / 65.
+//  * Q6_K against the streaming kernel: two tokens 3072x2048 of 8 10.9 / 9.0,
+//    14336x4096 38 / 31, 4096x14336 42.7 / 44.5; three 14336x4096 50 / 53.
+static bool cw_moe_wins(int fmt, const MoeArgs & a) {
+    const uint64_t weights = (uint64_t)a.rows * a.cols;
+    const uint32_t pairs = a.ntok * a.top_k, cus = (uint32_t)num_cus();
+    if (fmt == FMT_Q4_K || a.cols < 256 || a.cols > 8192 || pairs == 0) return true;
+    if (fmt == FMT_Q6_K) return a.ntok > 2 || cus % pairs || weights < (1u << 21);
+    // that launch's workgroups for a pair: no more than there are chunks of rows
+    const uint32_t rpc = 32 / (a.cols >> 8), chunks = (a.rows + rpc - 1) / rpc;
+    uint32_t per = (cus + pairs - 1) / pairs;
+    if (per > chunks) per = chunks;
+    if (per * pairs > cus) return true;
+    float routed = 1.f;                                           // experts that some token takes, on average
+    for (uint32_t t = 0; t < a.ntok; ++t) routed *= 1.f - (float)a.top_k / (float)a.n_expert;
+    routed = (float)a.n_expert * (1.f - routed);
+    float most;
+    if (weights <= (1u << 18) && pairs <= 64) return false;
+    if (cw_iq(fmt)) most = weights <= (1u << 23) ? 1.6f : weights <= (1u << 24) ? 1.47f : 1.2f;
+    else most = weights <= (1u << 18) ? 1.6f : weights > (1u << 23) ? 1.12f : pairs <= 32 ? 1.53f : 1.3f;
+    return (float)pairs > most * routed;
+}
+int launch_moe_cw(int fmt, const MoeArgs & a, hipStream_t s, bool any) {
+    if (!cw_on(fmt) || (!any && tune().cw == 1 && !cw_moe_wins(fmt, a))) return FLH_ERR_UNSUPPORTED;
     const uint64_t pairs = (uint64_t)a.ntok * a.top_k;
     if (pairs > 256 || a.n_expert > 256 || !cw_takes(fmt, a.w, a.estride, a.x, a.xstride, (uint32_t)pairs, a.cols))
         return FLH_ERR_UNSUPPORTED;

@@ -720,6 +720,7 @@ int launch_moe_i8k(int fmt, const MoeArgs & a, hipStream_t s) {
     if (a.ntok > 1) rc = launch_moe_cw(fmt, a, s);
     if (rc != FLH_ERR_UNSUPPORTED) return rc;
     rc = launch_moe_kstream(fmt, a, s);
+    if (rc == FLH_ERR_UNSUPPORTED && a.ntok > 1) rc = launch_moe_cw(fmt, a, s, true);
     if (rc != FLH_ERR_UNSUPPORTED) return rc;
     if (fmt == FMT_Q4_K) return launch_moe_t<FMT_Q4_K, 4>(a, s);
     if (fmt == FMT_Q6_K) return launch_moe_t<FMT_Q6_K, 4>(a, s);

@@ -176,8 +176,9 @@ int launch_moe_i8k(int fmt, const MoeArgs & a, hipStream_t s);
 // cores, one accumulator chain per wave (flh_dot_cw.hip); FLH_ERR_UNSUPPORTED
 // (nothing launched) if the kernel does not take the shape or another is faster
 int launch_dot_cw(int fmt, const DotArgs & a, hipStream_t s);
-// grouped experts on the same kernel (several tokens)
-int launch_moe_cw(int fmt, const MoeArgs & a, hipStream_t s);
+// grouped experts on the same kernel (any: also where another is faster, for
+// shapes that one declined)
+int launch_moe_cw(int fmt, const MoeArgs & a, hipStream_t s, bool any = false);
 // LDS-staged grouped expert kernel; FLH_ERR_UNSUPPORTED if it does not fit
 int launch_moe_kstream(int fmt, const MoeArgs & a, hipStream_t s);
 int launch_moe_sbl(int fmt, const MoeArgs & a, hipStream_t s);

@@ -1,10 +1,10 @@
 """The lines between the chain-per-wave kernel and the formats' other kernels: on
 either side of each, the default routing, the kernel by force (FLH_CW=2) and
-without it (FLH_CW=0) give the oracle's bits."""
+without it (FLH_CW=0) give the oracle's bits, dense and grouped."""
 import numpy as np
 import pytest
 
-from oracle import Q8_0, Q5_0, Q4_K, Q6_K, IQ2_XXS, IQ3_XXS, col_stride_floats
+from oracle import Q8_0, Q5_0, Q4_K, Q6_K, IQ2_XXS, IQ3_XXS, col_stride_floats, row_bytes
 from util import activations, sane_rows, tuned
 from test_gpu_parity import bits, dev_cols, say
 
@@ -36,4 +36,35 @@ def test_dense(flh, orc, gpu, fmt, rows, cols, nx):
         dy = flh.DeviceBuffer.from_array(y0, gpu)
         with tuned(flh, FLH_CW=mode):
             flh.stream_dot(fmt, dw, rows, cols, dx, dy, gpu, nx=nx, xstride=st, ystride=rows, i8_mask=0x7F)
+            assert np.array_equal(bits(dy.download(np.float32, y0.size, gpu)), bits(want)), mode
+
+
+@pytest.mark.parametrize("fused", [False, True])
+@pytest.mark.parametrize("rows,cols,ntok,top_k,experts", [
+    (64, 1024, 16, 4, 16), (256, 1024, 16, 8, 64), (257, 1024, 8, 2, 8), (1024, 2048, 2, 2, 8), (300, 2048, 4, 2, 8),
+    (300, 2048, 8, 4, 64), (300, 2048, 3, 6, 64), (40, 8448, 2, 2, 4), (600, 1280, 2, 4, 16)])
+@pytest.mark.parametrize("fmt", [Q8_0, Q5_0, Q6_K, IQ2_XXS, IQ3_XXS])
+def test_grouped(flh, orc, gpu, fmt, rows, cols, ntok, top_k, experts, fused):
+    say("cw moe routes", fmt, rows, cols, ntok, top_k, experts, fused)
+    rng = np.random.default_rng(fmt + rows + cols + ntok)
+    pairs, eb = ntok * top_k, rows * row_bytes(fmt, cols)
+    logits = rng.standard_normal((ntok, experts)).astype(np.float32)
+    ids = np.argsort(-logits, axis=1, kind="stable")[:, :top_k].astype(np.uint32)
+    w, xs = sane_rows(fmt, experts * rows, cols, rng), activations(ntok, cols, rng, outliers=True)
+    y0 = rng.standard_normal(pairs * rows).astype(np.float32)
+    st = (col_stride_floats(cols) + 3) & ~3
+    dx, _ = dev_cols(flh, gpu, xs, st)
+    flh.act_q8(dx, cols, gpu, nx=ntok, xstride=st)
+    dw, di, dg = flh.DeviceBuffer.from_array(w, gpu), flh.DeviceBuffer.from_array(ids, gpu), flh.DeviceBuffer(4 * pairs)
+    dl, want, xq = flh.DeviceBuffer.from_array(logits, gpu), y0.copy(), orc.act_q8_cols(xs, st)
+    for i, e in enumerate(ids.reshape(-1)):
+        orc.stream_dot(fmt, w[e * eb:(e + 1) * eb], rows, cols, xq[i // top_k * st:], want[i * rows:(i + 1) * rows], xstride=st,
+                       ystride=rows, i8_mask=0x7F)
+    for mode in "102":
+        dy = flh.DeviceBuffer.from_array(y0, gpu)
+        with tuned(flh, FLH_CW=mode):
+            if fused:
+                flh.router_moe_dot(fmt, dw, eb, rows, cols, dl, ntok, experts, top_k, 1, 1.0, di, dg, dx, st, False, dy, rows, gpu)
+            else:
+                flh.moe_dot(fmt, dw, eb, rows, cols, di, ntok, top_k, experts, dx, st, False, dy, rows, gpu)
             assert np.array_equal(bits(dy.download(np.float32, y0.size, gpu)), bits(want)), mode
