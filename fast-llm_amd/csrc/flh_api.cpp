@@ -337,18 +337,21 @@ struct flh_arena {
     size_t cap, used;
 };
 
-// A captured graph: the runtime's executable form and, for a chain of at most
-// five kernels, the kernels themselves, which are launched one by one on a
-// stream of this library's own (see flh_graph_launch).  The runtime's graph
-// launch adds about 6 us on the device to every replay and 16-18 us on the
-// host; a launch costs 2.6 us of host time, more where many are queued or
-// follow a wait.  us a replay in a row / us a replay that is waited for, one by
-// one against the runtime's launch: 4 kernels that clear 4 KiB 10.6 / 19
-// against 17.7 / 35, 5 13.3 / 21 against 18.0 / 35, but 6 20.6 / 23 against
-// 17.5 / 35, 12 40 / 79 against 26.5 / 38; 5 dots of 4096x4096 Q8_0 30.2 / 41
-// against 34.3 / 45.  A decode pass of 12 kernels (2048 columns) takes 51 / 76
-// against 57 / 65: faster in a row, but a decoder waits for every pass.  So the
-// line is where both are faster for the shortest kernels.
+// A captured graph: the runtime's executable form and, for a short chain of
+// kernels, the kernels themselves, which are launched one by one on a stream of
+// this library's own (see flh_graph_launch).  The runtime's graph launch adds
+// about 6 us on the device to every replay and 16-18 us on the host; a launch
+// costs 2.6 us of host time, 4 where many are queued or follow a wait.  us a
+// replay in a row / us a replay that is waited for, one by one against the
+// runtime's launch: 4 kernels that clear 4 KiB 10.6 / 19 against 17.7 / 35, 5
+// 13.3 / 21 against 18.0 / 35, but 6 20.6 / 23 against 17.5 / 35, 12 40 / 79
+// against 26.5 / 38: up to 5 kernels of any length.  Up to 16 only where the
+// device stays behind the host, which the weights that they stream tell: from an
+// average of 12 MiB a kernel a replay in a row is faster throughout and one that
+// is waited for within 7 % either way.  12 dots of 3584x4096 Q8_0 71 / 83 against
+// 75 / 86, of 6144x4096 89 / 100 against 92 / 105; 12 kernels of a decode pass of
+// 4096 columns (Q4_K, 20 MiB) 75 / 95 against 81 / 90, of 2048 columns (5 MiB) 51 /
+// 76 against 57 / 65.
 namespace {
 struct graph_handle {
     hipGraphExec_t exec = nullptr;
@@ -356,13 +359,28 @@ struct graph_handle {
     int device = 0;
     std::vector<hipKernelNodeParams> chain;
 };
-constexpr size_t GRAPH_CHAIN_MAX = 5;
+constexpr size_t CHAIN_ANY = 5, CHAIN_MAX = 16;
+constexpr uint64_t CHAIN_BYTES = 12u << 20;
 
-// the nodes of g in order, if they are one chain of at most GRAPH_CHAIN_MAX kernels
+// The weight bytes of the dots that this thread issues into the capture that it
+// began last.
+struct capture_weights {
+    void * stream = nullptr;
+    uint64_t bytes = 0;
+};
+thread_local capture_weights g_capture;
+void note_weights(void * stream, uint64_t bytes) {
+    if (g_capture.stream == stream) g_capture.bytes += bytes;
+}
+void note_experts(void * stream, const MoeArgs & a, int fmt) {
+    note_weights(stream, (uint64_t)moe_rows(a) * a.rows * flh_row_bytes(fmt, a.cols));
+}
+
+// the nodes of g in order, if they are one chain of at most CHAIN_MAX kernels
 bool kernel_chain(hipGraph_t g, std::vector<hipKernelNodeParams> & out) {
     size_t n = 0, one = 1;
     hipGraphNode_t node;
-    if (hipGraphGetNodes(g, nullptr, &n) != hipSuccess || n == 0 || n > GRAPH_CHAIN_MAX) return false;
+    if (hipGraphGetNodes(g, nullptr, &n) != hipSuccess || n == 0 || n > CHAIN_MAX) return false;
     if (hipGraphGetRootNodes(g, nullptr, &one) != hipSuccess || one != 1) return false;
     if (hipGraphGetRootNodes(g, &node, &one) != hipSuccess) return false;
     out.clear();
@@ -556,6 +574,7 @@ int flh_event_destroy(void * e) { return e ? hip_check(hipEventDestroy((hipEvent
 int flh_graph_capture_begin(void * stream) {
     if (int rc = need_init()) return rc;
     const StreamTurn turn(stream);
+    g_capture = {stream, 0};
     return hip_check(hipStreamBeginCapture((hipStream_t)stream, hipStreamCaptureModeThreadLocal),
                      "hipStreamBeginCapture");
 }
@@ -576,7 +595,9 @@ int flh_graph_capture_end(void * stream, void ** graph_exec) {
         delete h;
         return rc;
     }
-    if (kernel_chain(g, h->chain)) {
+    const uint64_t weights = g_capture.stream == stream ? g_capture.bytes : 0;
+    g_capture = {};
+    if (kernel_chain(g, h->chain) && (h->chain.size() <= CHAIN_ANY || weights >= CHAIN_BYTES * h->chain.size())) {
         h->graph = g;
     } else {
         h->chain.clear();
@@ -635,6 +656,7 @@ int flh_stream_dot(int fmt, const void * w, uint64_t w_bytes, uint32_t rows, uin
     if (int rc = validate_dot(fmt, w, w_bytes, rows, cols, x, y, nx, id_slot, estride, ystride)) return rc;
     if (int rc = need_init()) return rc;
     const StreamTurn turn(stream);
+    note_weights(stream, w_bytes);
     DotArgs a{(const uint8_t *)w, id_slot, estride, x, y, rows, cols, nx, xstride, ystride};
     return dispatch_dot(fmt, a, fast, i8_mask, i8k_mask, (hipStream_t)stream);
 }
@@ -651,6 +673,7 @@ int flh_act_q8_stream_dot(int fmt, const void * w, uint64_t w_bytes, uint32_t ro
     if (int rc = need_init()) return rc;
     const StreamTurn turn(stream);
     hipStream_t s = (hipStream_t)stream;
+    note_weights(stream, w_bytes);
     DotArgs a{(const uint8_t *)w, id_slot, estride, x, y, rows, cols, nx, xstride, ystride};
     // Fused when every workgroup re-reading the fp32 column is cheaper than a
     // separate ACT_Q8 launch.
@@ -693,6 +716,7 @@ int flh_rmsnorm_stream_dot(int fmt, const void * w, uint64_t w_bytes, uint32_t r
     const float * xe = x + cols;
     const float * ye = (const float *)((const uint8_t *)xn + x_alloc_bytes(cols));
     if (x < ye && xn < xe) return set_error(FLH_ERR_ARG, "rmsnorm dot: xn overlaps x");
+    note_weights(stream, w_bytes);
     DotArgs a{(const uint8_t *)w, nullptr, 0, xn, y, rows, cols, 1u, 0, 0};
     return rmsnorm_dot(fmt, a, NormArgs{x, wnorm, eps}, fast, i8_mask, i8k_mask, (hipStream_t)stream);
 }
@@ -710,6 +734,8 @@ int flh_exec_tasks(const flh_task * t, uint32_t n, int fast, uint32_t i8_mask, u
     if (int rc = need_init()) return rc;
     const StreamTurn turn(stream);
     hipStream_t s = (hipStream_t)stream;
+    for (uint32_t i = 0; i < n; ++i)
+        if (t[i].kind == FLH_TASK_STREAM_DOT || t[i].kind == FLH_TASK_STREAM_DOT_IDX) note_weights(stream, t[i].w_bytes);
     for (uint32_t i = 0; i < n; ++i) {
         const flh_task & k = t[i];
         int rc = FLH_OK;
@@ -820,6 +846,7 @@ int flh_moe_dot(int fmt, const void * w, uint64_t estride, uint32_t rows, uint32
         return set_error(FLH_ERR_ARG, "moe_dot: expert stride smaller than one expert or misaligned");
     MoeArgs a{(const uint8_t *)w, estride, ids, x, y, rows, cols, ntok, top_k, n_expert, xstride, ystride,
               x_per_slot};
+    note_experts(stream, a, fmt);
     if (fmt == FLH_FMT_Q4_K || fmt == FLH_FMT_Q6_K) return launch_moe_i8k(fmt, a, (hipStream_t)stream);
     return launch_moe_b32(fmt, a, (hipStream_t)stream);
 }
@@ -843,6 +870,7 @@ int flh_router_moe_dot(int fmt, const void * w, uint64_t estride, uint32_t rows,
     hipStream_t s = (hipStream_t)stream;
     MoeArgs a{(const uint8_t *)w, estride, ids, x, y, rows, cols, ntok, top_k, n_expert, xstride, ystride,
               x_per_slot};
+    note_experts(stream, a, fmt);
     // routing inside the grouped kernels (one launch) where they take it
     if (n_expert <= 64 && top_k <= 8 && ntok * top_k <= 256) {
         MoeArgs f = a;

@@ -1,5 +1,5 @@
 """Captured graphs: short chains of kernels (launched one by one on replay), at
-and past the 5-kernel line, and a capture with a copy node (the runtime's
+and past the lines of 5 kernels and of 16 that stream many weights, and a capture with a copy node (the runtime's
 form).  Every replay equals the eager result, with eager work, a change of the
 inputs and synchronizations between the replays, on the captured stream and on
 another one."""
@@ -16,9 +16,18 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("layers,more,copy", [(0, 0, False), (1, 0, False), (1, 1, False), (1, 2, False), (2, 0, False),
                                               (1, 0, True), (5, 0, False), (5, 0, True), (6, 0, False), (9, 0, False)])
 def test_replays_equal_eager(flh, gpu, layers, more, copy):
+    replays(flh, gpu, layers, more, copy, 96, 512)
+
+
+@pytest.mark.parametrize("layers,more", [(2, 0), (5, 0), (5, 1)])
+def test_replays_of_large_matrices(flh, gpu, layers, more):
+    """Dots of 27 MiB each: chains of 7 and 16 kernels past 12 MiB a kernel, and one too long."""
+    replays(flh, gpu, layers, more, False, 12288, 4096)
+
+
+def replays(flh, gpu, layers, more, copy, rows, cols):
     """1 + 3 * layers + more launches (and a copy): zero, then ACT_Q8, dot, dot."""
     say("graph chain", layers, more, copy)
-    rows, cols = 96, 512
     rng = np.random.default_rng(layers)
     st = col_stride_floats(cols)
     xb = np.zeros(st, np.float32)
