@@ -1,5 +1,7 @@
 // flh_dot_mfma.hip -- multi-column Q4_K x q8_K row-dots (speculative verify,
-// the shapes flh_dot_cw.hip leaves to it) on gfx950's int8 matrix cores.
+// the shapes flh_dot_cw.hip leaves to it: 9-16 columns of tall matrices, 5-8 of
+// tall ones whose rows end in part of a chunk there, 5-8 of few long rows) on
+// gfx950's int8 matrix cores.
 //
 // With several activation columns the per-lane VALU dot of the streaming
 // kernel (flh_dot_kstream.hip) becomes instruction-bound (about 300 wave
@@ -920,7 +922,6 @@ static int mf_launch_d(const DotArgs & a, uint32_t nrb, uint32_t grid, size_t sm
 
 size_t lds_limit();
 
-
 // LDS plan for NC columns: one workgroup per CU, batch of nrb rows (a multiple
 // of 16), ring depth D, whole activations or K halves (kh) when the whole
 // activations do not fit with a 16-row batch; FLH_ERR_UNSUPPORTED if neither
@@ -928,7 +929,7 @@ size_t lds_limit();
 template <int NC>
 static int mf_plan_kh(uint32_t rows, uint32_t nsb, uint32_t G, uint32_t & nrb, int & D, bool & kh, size_t & smb,
                       bool * xc = nullptr, bool * own = nullptr) {
-    const size_t lim = lds_limit() - 4096;
+    const size_t lim = lds_limit() - 4096;                    // (the plans were measured within this)
     const uint32_t rpw = (rows + G - 1) / G;
     // a batch's old y values are one 64-float DMA per wave: nrb * NC <= 512
     nrb = ((rpw + 15) / 16) * 16;

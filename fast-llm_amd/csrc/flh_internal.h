@@ -172,8 +172,8 @@ int launch_dot_fast_f32(int fmt, const DotArgs & a, hipStream_t s);
 int launch_dequant(int fmt, const uint8_t * w, uint32_t rows, uint32_t cols,
                    float * out, hipStream_t s);
 int launch_moe_i8k(int fmt, const MoeArgs & a, hipStream_t s);
-// 1..16 columns of Q8_0, Q5_0 (q8_1), 2..16 of Q4_K, Q6_K (q8_K) on the int8 matrix
-// cores, one accumulator chain per wave (flh_dot_cw.hip); FLH_ERR_UNSUPPORTED
+// 1..16 columns of Q8_0, Q5_0, IQ2_XXS, IQ3_XXS (q8_1), 2..16 of Q4_K, Q6_K (q8_K) on
+// the int8 matrix cores, one accumulator chain per wave (flh_dot_cw.hip); FLH_ERR_UNSUPPORTED
 // (nothing launched) if the kernel does not take the shape or another is faster
 int launch_dot_cw(int fmt, const DotArgs & a, hipStream_t s);
 // grouped experts on the same kernel (any: also where another is faster, for

@@ -1,5 +1,6 @@
 """GPU parity of the multi-column Q4_K kernel on the int8 matrix cores
-(flh_dot_mfma.hip, used by STREAM_DOT for 2..16 Q4_K columns).
+(flh_dot_mfma.hip: 2..16 Q4_K columns; every run here keeps off the kernel
+that most shapes take by default, FLH_CW=0).
 
 Bar: bitwise against the oracle (the reference's fl_dot_i8k_q4_K per column,
 src/runtime/quants.h:538-561), at the speculative-verify shapes of the
@@ -20,6 +21,12 @@ from util import sane_rows, activations, tuned
 from test_gpu_parity import run_dot, bits, say
 
 pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(autouse=True)
+def on_this_kernel(flh, gpu):
+    with tuned(flh, FLH_CW="0"):
+        yield
 
 
 @pytest.mark.parametrize("rows,cols,nx", [

@@ -278,11 +278,10 @@ def test_router_moe_dot_fused_equals_separate(flh, gpu, fmt, ntok, rows, cols, p
 
 
 @pytest.mark.parametrize("ntok,rows,cols,per_slot", [(8, 300, 4096, False), (6, 130, 2816, True)])
-def test_grouped_expert_dot_k_halves_bitwise(flh, orc, gpu, ntok, rows, cols, per_slot):
-    """The grouped matrix-core kernel with K halves forced (the mode wide
-    expert inputs take when the whole activations do not fit LDS), bitwise."""
+def test_grouped_expert_dot_streaming_bitwise(flh, orc, gpu, ntok, rows, cols, per_slot):
+    """The grouped streaming kernel (several tokens, off the matrix cores), bitwise."""
     from util import tuned
-    with tuned(flh, FLH_MFMA_TUNE="2,0,1"):
+    with tuned(flh, FLH_CW="0"):
         grouped_dot_case(flh, orc, gpu, Q4_K, ntok, rows, cols, per_slot)
 
 

@@ -59,11 +59,10 @@ CASES = [
 
 
 @pytest.mark.parametrize("ntok", [3, 8])
-def test_moe_register_sums_keep_bits(flh, gpu, ntok):
-    """The grouped matrix-core expert dots with register accumulators (the
-    default) and with parked terms and a fold pass (FLH_MFMA_OWN=0) give the
-    same bits for every (token, slot) pair."""
-    say("tuning moe own", ntok)
+def test_moe_matrix_cores_keep_bits(flh, gpu, ntok):
+    """The grouped expert dots on the matrix cores (the default) and on the
+    streaming kernel (FLH_CW=0) give the same bits for every (token, slot) pair."""
+    say("tuning moe cw", ntok)
     E, K, rows, cols = 6, 2, 1500, 4096
     rng = np.random.default_rng(ntok)
     from oracle import row_bytes
@@ -77,7 +76,7 @@ def test_moe_register_sums_keep_bits(flh, gpu, ntok):
     dw = flh.DeviceBuffer.from_array(w, gpu)
     did = flh.DeviceBuffer.from_array(ids, gpu)
     out = []
-    for env in ({}, {"FLH_MFMA_OWN": "0"}):
+    for env in ({}, {"FLH_CW": "0"}):
         dy = flh.DeviceBuffer(ntok * K * rows * 4)
         dy.zero(gpu)
         with tuned(flh, **env):
@@ -92,9 +91,12 @@ def test_switch_keeps_bits(flh, orc, gpu, name, value, fmt, rows, cols, nx, mis,
     rng = np.random.default_rng(rows + cols + nx)
     w = sane_rows(fmt, rows, cols, rng)
     xs = activations(nx, cols, rng, outliers=True)
-    base, want = run(flh, orc, gpu, fmt, w, rows, cols, xs, mis, fused)
+    # a switch of the Q4_K matrix-core kernel: both runs on that kernel
+    here = {"FLH_CW": "0"} if name.startswith("FLH_MFMA") else {}
+    with tuned(flh, **here):
+        base, want = run(flh, orc, gpu, fmt, w, rows, cols, xs, mis, fused)
     assert np.array_equal(bits(base), bits(want))
-    with tuned(flh, **{name: value}):
+    with tuned(flh, **here, **{name: value}):
         got, _ = run(flh, orc, gpu, fmt, w, rows, cols, xs, mis, fused)
     assert np.array_equal(bits(got), bits(want))
 
