@@ -663,7 +663,7 @@ __global__ __launch_bounds__(64 * CW_WAVES, 4) void k_moe_cw(MoeArgs a) {
 // ----------------------------------------------------------------- launch --
 static bool cw_takes(int fmt, const void * w, uint64_t estride, const void * x, uint32_t xstride, uint32_t ncol,
                      uint32_t cols) {
-    if (cols == 0 || (cols & 255) || ((uintptr_t)x & 3)) return false;
+    if (cols == 0 || cols > 16384 || (cols & 255) || ((uintptr_t)x & 3)) return false;   // (longer rows are refused everywhere)
     if (fmt != FMT_Q4_K && fmt != FMT_Q6_K && (((uintptr_t)x & 15) || (xstride & 3))) return false;
     // 32-bit lane offsets
     if ((uint64_t)ncol * xstride * 4 + x_alloc_bytes(cols) >= (1ull << 32) || 16ull * cols * 2 >= (1ull << 32)) return false;

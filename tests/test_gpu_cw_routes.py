@@ -39,6 +39,23 @@ def test_dense(flh, orc, gpu, fmt, rows, cols, nx):
             assert np.array_equal(bits(dy.download(np.float32, y0.size, gpu)), bits(want)), mode
 
 
+@pytest.mark.parametrize("fmt", [Q8_0, Q5_0, Q4_K, Q6_K, IQ2_XXS, IQ3_XXS])
+def test_longer_rows_are_refused(flh, gpu, fmt):
+    """More than 16384 columns are refused whatever the rows and columns (as
+    every other kernel of these formats refuses them), dense and grouped."""
+    say("cw refused", fmt)
+    cols, rows, E = 16640, 4200, 2
+    w, x = flh.DeviceBuffer(rows * row_bytes(fmt, cols)), flh.DeviceBuffer(16 * flh.x_alloc_bytes(cols) + 256)
+    y, ids = flh.DeviceBuffer(16 * rows * 4), flh.DeviceBuffer.from_array(np.array([0, 1, 1, 0], np.uint32), gpu)
+    st = (col_stride_floats(cols) + 3) & ~3
+    for r, nx in ((rows, 1), (rows, 2), (rows, 8), (33, 4), (rows, 16)):
+        with pytest.raises(flh.FlhError):
+            flh.stream_dot(fmt, w, r, cols, x, y, gpu, nx=nx, xstride=st, ystride=r, i8_mask=0x7F)
+    for n, k in ((2, 2), (2, 1)):
+        with pytest.raises(flh.FlhError):
+            flh.moe_dot(fmt, w, 16 * row_bytes(fmt, cols), 16, cols, ids, n, k, E, x, st, False, y, 16, gpu)
+
+
 @pytest.mark.parametrize("fused", [False, True])
 @pytest.mark.parametrize("rows,cols,ntok,top_k,experts", [
     (64, 1024, 16, 4, 16), (256, 1024, 16, 8, 64), (257, 1024, 8, 2, 8), (1024, 2048, 2, 2, 8), (300, 2048, 4, 2, 8),
