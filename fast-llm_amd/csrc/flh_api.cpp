@@ -198,18 +198,19 @@ static int dispatch_dot(int fmt, const DotArgs & a, int fast, uint32_t i8_mask, 
 // Otherwise the routed superblock-per-lane launch, one workgroup row per
 // (token, slot) pair (the reference runs these per pair too,
 // src/model/decoder.cpp:941-996).  Shapes its LDS plan cannot hold (rows of more
-// than ~14.5K columns) run on the matrix cores too; what neither takes (weights
-// or x not 16-byte aligned) runs as the reference's own per-pair STREAM_DOT_IDX
-// tiles, the id read on the device, on the q8_1 int8 path the routed launch
-// computes (same bits); there the ids must be < n_expert, as ROUTER_SEL writes
-// them (the routed launch also skips larger ones).
+// than ~14.5K columns, IQ rows of a number of columns that is no multiple of
+// 2048) run on the matrix cores too.  What neither takes (weights or x not
+// 16-byte aligned) and a single pair (IQ2_XXS 256x1024 3.7 us, 5.1 there) run as
+// the reference's own per-pair STREAM_DOT_IDX tiles, the id read on the device, on
+// the q8_1 int8 path the routed launch computes (same bits); there the ids must be
+// < n_expert, as ROUTER_SEL writes them (the routed launch also skips larger ones).
 static int launch_moe_b32(int fmt, const MoeArgs & a, hipStream_t s) {
     if (a.rows == 0 || a.ntok == 0 || a.top_k == 0) return FLH_OK;
     if (a.ntok * a.top_k > 256) return set_error(FLH_ERR_UNSUPPORTED, "moe: ntok*top_k > 256");
     int rc = FLH_ERR_UNSUPPORTED;
     if (a.ntok > 1) rc = launch_moe_cw(fmt, a, s);
     if (rc == FLH_ERR_UNSUPPORTED) rc = launch_moe_sbl(fmt, a, s);
-    if (rc == FLH_ERR_UNSUPPORTED) rc = launch_moe_cw(fmt, a, s, true);
+    if (rc == FLH_ERR_UNSUPPORTED && a.ntok * a.top_k > 1) rc = launch_moe_cw(fmt, a, s, true);
     if (rc != FLH_ERR_UNSUPPORTED) return rc;
     for (uint32_t p = 0; p < a.ntok * a.top_k; ++p) {
         const uint32_t xi = a.x_per_slot ? p : p / a.top_k;
@@ -881,7 +882,7 @@ int flh_router_moe_dot(int fmt, const void * w, uint64_t estride, uint32_t rows,
         int rc = FLH_ERR_UNSUPPORTED;
         if (ntok > 1) rc = launch_moe_cw(fmt, f, s);
         if (rc == FLH_ERR_UNSUPPORTED && (ntok == 1 || !kf) && tune().sbl) rc = launch_moe_sbl(fmt, f, s);
-        if (rc == FLH_ERR_UNSUPPORTED && !kf) rc = launch_moe_cw(fmt, f, s, true);
+        if (rc == FLH_ERR_UNSUPPORTED && !kf && ntok * top_k > 1) rc = launch_moe_cw(fmt, f, s, true);
         if (rc == FLH_ERR_UNSUPPORTED && kf) rc = launch_moe_kstream(fmt, f, s);
         if (rc == FLH_ERR_UNSUPPORTED && ntok > 1 && kf) rc = launch_moe_cw(fmt, f, s, true);
         if (rc != FLH_ERR_UNSUPPORTED) return rc;

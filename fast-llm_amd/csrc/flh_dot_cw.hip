@@ -716,7 +716,7 @@ template <int FMT> static int cw_launch(const DotArgs & a, hipStream_t s) {
 //  * Q8_0 and Q5_0 against k_dot_sbl_nx (rows of up to 8192 columns) and the
 //    register kernel.  2 columns Q8_0 14336x4096 15.3 / 14.4, 4096x8192 9.9 / 11.5,
 //    2048x8192 9.4 / 8.1, 4096x14336 14.2 / 20.1, Q5_0 14336x4096 12.3 / 14.2,
-//    2048x4096 6.5 / 5.8; 4 columns Q8_0 1024x4096 6.4 / 6.4, 14336x4096 15.7 /
+//    2048x4096 6.5 / 5.8; 4 columns Q8_0 1024x1792 5.1 / 4.8, 14336x4096 15.7 /
 //    18.1; 5 columns Q5_0 512x8192 11.3 / 10.1 (8 columns 11.4 / 11.7), Q8_0 256x6144
 //    8.9 / 8.1; 16 columns 14336x4096 20 / 52.  One column against k_dot_sbl: rows
 //    wider than its one pass per lane group holds well, Q8_0 4096x14336 14.3 / 18.6,
@@ -730,7 +730,8 @@ template <int FMT> static int cw_launch(const DotArgs & a, hipStream_t s) {
 //    / 12.2), 1024x8192 12.9 / 11.9; 16 columns 14336x4096 25.7 / 42.6.  Other row
 //    lengths: 2 columns 1024x2816 5.9 / 5.8, 2048x2816 6.3 / 7.9, 1024x14336 15.8 /
 //    14.8; 4 columns 256x1792 IQ3_XXS 4.9 / 4.5, 512x2816 5.8 / 5.7; 3840x3840 with 1
-//    / 16 6.5 / 7.7, 10.2 / 44; one column of few rows, 1024x2816: 5.4 / 5.1.
+//    / 16 6.5 / 7.7, 10.2 / 44; one column of few rows, 1024x2816 5.4 / 5.1,
+//    2048x16384 17.4 / 15.2, 256x16384 16.9 / 10.8.
 static bool cw_wins(int fmt, uint32_t rows, uint32_t cols, uint32_t nx) {
     const uint32_t T = (rows + 15) / 16, cus = (uint32_t)num_cus();
     const bool half = 2 * T <= cus, quarter = 4 * T <= cus, sixteenth = 16 * T <= cus;   // of the chip, at most
@@ -747,7 +748,7 @@ static bool cw_wins(int fmt, uint32_t rows, uint32_t cols, uint32_t nx) {
     }
     if (cw_iq(fmt)) {
         const bool sbl = !(cols & 2047) && cols <= 8192;
-        if (nx == 1) return cols > 16128 || ((cols & 2047) && rows >= 2048);
+        if (nx == 1) return ((cols & 2047) || cols > 16128) && (cols > 8192 ? !half : rows >= 2048);
         if (nx == 2) return sbl ? rows > 16384 && cols > 2048 : !(quarter && cols > 1024);
         if (nx <= 4 && sbl) return !(half && cols > 2048);
         if (nx <= 4) return !(sixteenth && cols > 1024) && !((cols > 8192 ? quarter : 5 * T <= cus) && cols > 2048);
@@ -755,7 +756,7 @@ static bool cw_wins(int fmt, uint32_t rows, uint32_t cols, uint32_t nx) {
     }
     if (nx == 1) return cols > 4096 && T >= cus;
     if (nx == 2 && half && cols > 2048 && cols <= 8192) return false;
-    if (nx <= 4 && quarter && cols > 2048) return false;
+    if (nx <= 4 && quarter && cols > (fmt == FMT_Q8_0 && nx > 2 ? 1536u : 2048u)) return false;
     if (nx > 4 && nx <= 8 && sixteenth && cols > 4096 && cols <= 6144) return false;
     if (fmt == FMT_Q5_0 && (nx == 5 || nx == 6) && quarter && cols > 4096 && cols <= 8192) return false;
     return nx > 2 || fmt == FMT_Q5_0 || cols > 4096;

@@ -741,17 +741,18 @@ __global__ void k_dot_canon(int fmt, DotArgs a) {
 // workgroup; us there / here).  A workgroup costs about 0.65 ns of the chip
 // however short its row: it wins where the rows are few (the chip is filled sooner)
 // or long.  One column: 8x4096 10.2 / 3.9, 2048x64 4.0 / 3.7, 4096x64 4.1 / 4.9,
-// 65536x256 20 / 47; 4096x768 5.5 / 5.5, 8192x768 7.7 / 9.4, 16384x1024 18.5 / 17.5,
+// 65536x256 20 / 47; 4096x768 5.5 / 6.0, 4096x1024 7.8 / 6.7, 16384x1024 18.5 / 17.5,
 // 32768x1024 30.9 / 31.7, 65536x1536 69 / 73; 65536x2048 93 / 85, 262144x2048 337 /
 // 330, 262144x4096 764 / 677.  Several: 64x2048 with 4 columns 14.3 / 3.6, with 16 56
-// / 3.8, 2048x1024 with 3 / 4 9.0 / 7.8, 10.2 / 8.1, 2048x512 with 2 / 3 5.5 / 4.7, 6.7 /
-// 6.7, 2048x64 with 2 / 3 / 4 4.9 / 4.6, 5.1 / 6.5, 5.9 / 6.7, 1280x64 with 3 5.1 / 5.1;
+// / 3.8, 2048x1024 with 3 / 4 9.0 / 7.8, 10.2 / 8.1, 2048x512 with 2 / 3 5.5 / 4.7, 6.4 /
+// 6.9, 1281x512 with 3 6.3 / 5.4, 2048x64 with 2 / 3 / 4 4.9 / 4.6, 5.1 / 6.5, 5.9 / 6.7, 1280x64 with 3 5.1 / 5.1;
 // past 2048 workgroups 4096x4096 with 4 29 / 35, 16384x1024 with 4 21 / 55.  (A launch
 // holds fewer than 2^32 threads: 2^24 rows are k_dot_f32row's.)
 static bool f32_small(uint32_t rows, uint32_t cols, uint32_t nx) {
     if (rows >= (1u << 24)) return false;
-    if (nx == 1) return rows <= 2048 || cols >= 2048 || (cols >= 1024 ? rows <= 16384 : cols >= 768 && rows <= 4096);
-    return (uint64_t)rows * ((nx + 3) / 4) <= (cols < 512 && (nx == 3 || nx == 4) ? 1280u : 2048u);
+    if (nx == 1) return rows <= 2048 || cols >= 2048 || (cols >= 1024 && rows <= 16384);
+    const uint32_t most = nx == 3 && cols >= 512 && cols < 1280 ? 1536u : cols < 512 && (nx == 3 || nx == 4) ? 1280u : 2048u;
+    return (uint64_t)rows * ((nx + 3) / 4) <= most;
 }
 
 static int launch_f32(bool fast, int fmt, const DotArgs & a, hipStream_t s) {

@@ -18,7 +18,8 @@ DENSE = [(Q4_K, 16400, 768, 9), (Q4_K, 8200, 1280, 9), (Q4_K, 20500, 1280, 5), (
          (Q5_0, 1024, 8192, 6), (Q5_0, 1025, 8192, 5), (Q5_0, 1024, 8192, 7),
          (IQ2_XXS, 1024, 1280, 2), (IQ2_XXS, 1025, 1280, 2), (IQ3_XXS, 16400, 4096, 2), (IQ2_XXS, 2048, 4096, 4),
          (IQ3_XXS, 2049, 4096, 3), (IQ2_XXS, 2048, 8192, 6), (IQ3_XXS, 2048, 8192, 7), (IQ2_XXS, 256, 1280, 3),
-         (IQ3_XXS, 816, 2304, 4), (IQ2_XXS, 817, 2304, 4), (IQ3_XXS, 1024, 8448, 3), (IQ2_XXS, 1025, 8448, 4)]
+         (IQ2_XXS, 2048, 16384, 1),
+         (IQ3_XXS, 2049, 16384, 1), (IQ2_XXS, 2048, 8448, 1), (IQ3_XXS, 816, 2304, 4), (IQ2_XXS, 817, 2304, 4), (IQ3_XXS, 1024, 8448, 3), (IQ2_XXS, 1025, 8448, 4)]
 
 
 @pytest.mark.parametrize("fmt,rows,cols,nx", DENSE)

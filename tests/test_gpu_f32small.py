@@ -13,7 +13,7 @@ pytestmark = pytest.mark.gpu
 CASES = [(1, 16, 1), (3, 15, 2), (5, 64, 4), (7, 4095, 1), (2, 4096, 5), (9, 4097, 3), (4, 4112, 16), (3, 8192, 4),
          (2, 12289, 2), (64, 2048, 8), (512, 272, 16), (513, 272, 16), (2048, 48, 3), (2049, 48, 3), (5000, 512, 1),
          # either side of the routing lines: rows and lengths of one column, narrow rows of several
-         (2048, 100, 1), (2049, 100, 1), (4096, 768, 1), (4097, 768, 1), (4096, 767, 1), (16384, 1024, 1), (16385, 1024, 1),
+         (2048, 100, 1), (2049, 100, 1), (4096, 768, 1), (4096, 1024, 1), (1536, 512, 3), (1537, 1276, 3), (2048, 1280, 3), (16384, 1024, 1), (16385, 1024, 1),
          (20000, 2047, 1), (20000, 2048, 1), (1280, 500, 4), (1281, 500, 3), (1281, 512, 4), (2048, 512, 3)]
 
 
