@@ -35,9 +35,10 @@
 // scales had to be transposed per group, eight lane-row swaps: Q8_0 28672x4096
 // with 16 columns 34.6 -> 32.8 us, IQ2_XXS 4096x14336 29.0 -> 25.4, Q4_K 16.4 ->
 // 14.9, Q6_K vocabulary 128256x4096 with 5 / 16 columns 89.9 -> 88.9, 120 -> 114.
-// A lane reads one block's contiguous bytes, which for the 32-weight formats is
-// free of bank conflicts; 8 bytes of every block per lane (a plain A operand)
-// took 742 LDS cycles per chunk instead of about 140.
+// A lane reads one block's contiguous bytes; 8 bytes of every block per lane (a
+// plain A operand) took 742 LDS cycles per chunk instead of about 140.  (Rows r and
+// r + 8 of a Q8_0 or Q6_K stage share banks: 65 % of the LDS-active cycles are
+// conflicts, about 540 cycles a wave of Q8_0 14336x4096 with 4 columns; Q4_K 37 %.)
 //
 // IQ2_XXS / IQ3_XXS: 1024 columns a chunk, 8 blocks per wave in two halves that
 // run as Q8_0's; a lane expands its block from the codebook and a table of sign
