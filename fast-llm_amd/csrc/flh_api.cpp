@@ -346,13 +346,16 @@ struct flh_arena {
 // replay in a row / us a replay that is waited for, one by one against the
 // runtime's launch: 4 kernels that clear 4 KiB 10.6 / 19 against 17.7 / 35, 5
 // 13.3 / 21 against 18.0 / 35, but 6 20.6 / 23 against 17.5 / 35, 12 40 / 79
-// against 26.5 / 38: up to 5 kernels of any length.  Up to 16 only where the
-// device stays behind the host, which the weights that they stream tell: from an
-// average of 12 MiB a kernel a replay in a row is faster throughout and one that
-// is waited for within 7 % either way.  12 dots of 3584x4096 Q8_0 71 / 83 against
-// 75 / 86, of 6144x4096 89 / 100 against 92 / 105; 12 kernels of a decode pass of
-// 4096 columns (Q4_K, 20 MiB) 75 / 95 against 81 / 90, of 2048 columns (5 MiB) 51 /
-// 76 against 57 / 65.
+// against 26.5 / 38: up to 5 kernels of any length.  More only where the device
+// stays behind the host, which the weights that they stream tell.  6 and 7 are
+// faster either way with any dots to speak of (7 kernels of a decode pass of 1024
+// columns, Q4_K, 0.9 MiB a kernel, 25 / 38 against 32 / 43, of 3072 31 / 46 against
+// 38 / 47).  From 8 on a launch after a wait takes the host 4-5 us: from an average
+// of 12 MiB a kernel a replay in a row is faster throughout and one that is waited
+// for within 7 % either way (12 dots of 3584x4096 Q8_0 71 / 83 against 75 / 86, of
+// 6144x4096 89 / 100 against 92 / 105; 12 kernels of a decode pass of 4096 columns,
+// 20 MiB, 75 / 95 against 81 / 90), below it not (3072 columns, 10.6 MiB, 60 / 84
+// against 66 / 74; 2048 columns, 5 MiB, 51 / 76 against 57 / 65).
 namespace {
 struct graph_handle {
     hipGraphExec_t exec = nullptr;
@@ -360,8 +363,9 @@ struct graph_handle {
     int device = 0;
     std::vector<hipKernelNodeParams> chain;
 };
-constexpr size_t CHAIN_ANY = 5, CHAIN_MAX = 16;
-constexpr uint64_t CHAIN_BYTES = 12u << 20;
+constexpr size_t CHAIN_MAX = 16;
+// the average of weight bytes a kernel from which a chain of n is launched so
+constexpr uint64_t chain_weights(size_t n) { return n <= 5 ? 0 : n <= 7 ? 512u << 10 : 12u << 20; }
 
 // The weight bytes of the dots that this thread issues into the capture that it
 // began last.
@@ -598,7 +602,7 @@ int flh_graph_capture_end(void * stream, void ** graph_exec) {
     }
     const uint64_t weights = g_capture.stream == stream ? g_capture.bytes : 0;
     g_capture = {};
-    if (kernel_chain(g, h->chain) && (h->chain.size() <= CHAIN_ANY || weights >= CHAIN_BYTES * h->chain.size())) {
+    if (kernel_chain(g, h->chain) && weights >= chain_weights(h->chain.size()) * h->chain.size()) {
         h->graph = g;
     } else {
         h->chain.clear();

@@ -182,9 +182,9 @@ int flh_event_destroy(void * event);
  *
  * A replay is one operation of its stream: work that other threads issue there
  * through this library comes before or after all of it.  On a stream of
- * flh_stream_create a chain of at most 5 kernels, or of 16 that stream 12 MiB of
- * weights each on average, is replayed kernel by kernel (less idle time on the
- * device; 2.6 to 4 us of the caller's time per kernel).  What other code issues
+ * flh_stream_create a short chain of kernels (at most 5, 7 with 0.5 MiB of
+ * weights each on average, 16 with 12 MiB) is replayed kernel by kernel (less idle
+ * time on the device; 2.6 to 4 us of the caller's time per kernel).  What other code issues
  * there directly (a HIP call on the handle) from another thread at the same time
  * may then fall between two of the kernels, and a replay that fails may have run
  * in part.  On any other stream, and for any other graph, a replay is the

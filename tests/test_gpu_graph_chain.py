@@ -1,5 +1,5 @@
 """Captured graphs: short chains of kernels (launched one by one on replay), at
-and past the lines of 5 kernels and of 16 that stream many weights, and a capture with a copy node (the runtime's
+and past the lines of 5 kernels, 7 that stream some weights and 16 that stream many, and a capture with a copy node (the runtime's
 form).  Every replay equals the eager result, with eager work, a change of the
 inputs and synchronizations between the replays, on the captured stream and on
 another one."""
@@ -19,10 +19,12 @@ def test_replays_equal_eager(flh, gpu, layers, more, copy):
     replays(flh, gpu, layers, more, copy, 96, 512)
 
 
-@pytest.mark.parametrize("layers,more", [(2, 0), (5, 0), (5, 1)])
-def test_replays_of_large_matrices(flh, gpu, layers, more):
-    """Dots of 27 MiB each: chains of 7 and 16 kernels past 12 MiB a kernel, and one too long."""
-    replays(flh, gpu, layers, more, False, 12288, 4096)
+@pytest.mark.parametrize("layers,more,rows", [(1, 2, 1024), (2, 0, 1024), (2, 1, 1024), (2, 1, 12288), (5, 0, 12288),
+                                              (5, 1, 12288)])
+def test_replays_of_larger_matrices(flh, gpu, layers, more, rows):
+    """Dots of 2.3 and 27 MiB: chains of 6 and 7 kernels past 0.5 MiB a kernel and one
+    too long for that, of 8 and 16 past 12 MiB and one too long."""
+    replays(flh, gpu, layers, more, False, rows, 4096)
 
 
 def replays(flh, gpu, layers, more, copy, rows, cols):
